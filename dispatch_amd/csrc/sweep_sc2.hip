@@ -54,10 +54,10 @@ struct Row {
 // forms it (SRC/rt_solvers_mod.f90:355-370), and rc = 1/chi500; then 1/g500 of the
 // ghost plane.
 template <typename T>
-__global__ void __launch_bounds__(256) sc2_prep(const float *__restrict__ chi500,
-                                                const float *__restrict__ chi500_up,
-                                                const float *__restrict__ g500, T *__restrict__ dt500,
-                                                T *__restrict__ rc, int nxy, int nz, double dsup) {
+__global__ void __launch_bounds__(256) sc2_prep_kernel(const float *__restrict__ chi500,
+                                                       const float *__restrict__ chi500_up,
+                                                       const float *__restrict__ g500, T *__restrict__ dt500,
+                                                       T *__restrict__ rc, int nxy, int nz, double dsup) {
   const int64_t n = (int64_t)nxy * nz;
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n + nxy;
        i += (int64_t)gridDim.x * blockDim.x) {
@@ -79,20 +79,30 @@ __global__ void __launch_bounds__(256) sc2_prep(const float *__restrict__ chi500
   }
 }
 
+template <typename T>
+int sc2_prep(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const float *chi500, const float *chi500_up,
+             const float *g500, T *dt500, T *rc) {
+  const int64_t nxy = (int64_t)d->nx * d->ny, nprep = nxy * (d->nz + 1);
+  const double dsup = d->ds[2] / fabs(d->vec[2]);
+  const int blocks = (int)std::min<int64_t>((nprep + 255) / 256, 65536);
+  hipLaunchKernelGGL(sc2_prep_kernel<T>, dim3(blocks), dim3(256), 0, ctx->stream, chi500, chi500_up, g500, dt500,
+                     rc, (int)nxy, d->nz, dsup);
+  M3DRT_HIP(hipGetLastError());
+  return M3DRT_OK;
+}
+template int sc2_prep<float>(m3drt_ctx *, const m3drt_sweep_desc *, const float *, const float *, const float *,
+                             float *, float *);
+template int sc2_prep<double>(m3drt_ctx *, const m3drt_sweep_desc *, const float *, const float *, const float *,
+                              double *, double *);
+
 int sc2_prep_f32(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const float *chi500, const float *chi500_up,
                  const float *g500, float **dt500, float **rc) {
-  const int64_t nxy = (int64_t)d->nx * d->ny;
-  const size_t nprep = (size_t)nxy * (d->nz + 1);
+  const size_t nprep = (size_t)d->nx * d->ny * (d->nz + 1);
   const int st = ensure_scratch(ctx, sizeof(float) * 2 * nprep);
   if (st) return st;
   *dt500 = static_cast<float *>(ctx->scratch);
   *rc = *dt500 + nprep;
-  const double dsup = d->ds[2] / fabs(d->vec[2]);
-  const int blocks = (int)std::min<int64_t>(((int64_t)nprep + 255) / 256, 65536);
-  hipLaunchKernelGGL(sc2_prep<float>, dim3(blocks), dim3(256), 0, ctx->stream, chi500, chi500_up, g500, *dt500,
-                     *rc, (int)nxy, d->nz, dsup);
-  M3DRT_HIP(hipGetLastError());
-  return M3DRT_OK;
+  return sc2_prep<float>(ctx, d, chi500, chi500_up, g500, *dt500, *rc);
 }
 
 // Global inputs of one cell: opacity, source function, the cell's dt500 and
@@ -427,21 +437,38 @@ static int exact_dispatch(m3drt_ctx *ctx, const Sc2Args<T> &a, int L, int nt, in
   return exact_out<T, 30>(ctx, a, nt, nplanes, false);
 }
 
+// The limits of the workgroup-per-frequency kernels, which every route keeps: the
+// plane in the LDS, the strips in the workgroup, in-plane offsets in 32 bits.
+template <typename T>
+static int sc2_limits(m3drt_ctx *ctx, const m3drt_sweep_desc *d) {
+  const int nx = d->nx, ny = d->ny;
+  if (nx > 1024) return set_error(M3DRT_ELIMIT, "m3drt_sc_sweep: nx > 1024");
+  if ((size_t)nx * ny * sizeof(T) > (size_t)ctx->lds_max)
+    return set_error(M3DRT_ELIMIT, "m3drt_sc_sweep: the plane does not fit the LDS");
+  const int tmax = sizeof(T) == 8 ? 512 : 1024;
+  if (nx > tmax) return set_error(M3DRT_ELIMIT, "m3drt_sc_sweep: nx beyond the workgroup size");
+  const int smax = std::max(1, tmax / nx);
+  if ((ny + smax - 1) / smax > 32)
+    return set_error(M3DRT_ELIMIT, "m3drt_sc_sweep: ny too large for the strip mapping");
+  // in-plane offsets are 32-bit: every (x, y) offset of a cube and plane must fit
+  const uint64_t span = (uint64_t)(nx - 1) * d->cs_x + (uint64_t)(ny - 1) * d->cs_y;
+  const uint64_t gspan = (uint64_t)(nx - 1) * d->gs_x + (uint64_t)(ny - 1) * d->gs_y;
+  if ((span + 1) * sizeof(T) >= (1ull << 32) || (gspan + 1) * sizeof(T) >= (1ull << 32))
+    return set_error(M3DRT_ELIMIT, "m3drt_sc_sweep: in-plane offsets exceed 32 bits");
+  return M3DRT_OK;
+}
+
 template <typename T>
 static int run_sc2(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const m3drt_sweep_bufs *b) {
   const int nx = d->nx, ny = d->ny, nz = d->nz;
   const int64_t nxy = (int64_t)nx * ny;
-  if (nx > 1024) return set_error(M3DRT_ELIMIT, "m3drt_sc_sweep: nx > 1024");
   const size_t plane = (size_t)nxy * sizeof(T);
   const int nplanes = (int)std::min<size_t>(3, (size_t)ctx->lds_max / plane);
-  if (nplanes < 1) return set_error(M3DRT_ELIMIT, "m3drt_sc_sweep: the plane does not fit the LDS");
   // strips: as many rows per thread as the workgroup needs (1024 threads in FP32;
   // 512 in FP64, whose registers hold twice the bytes)
   const int tmax = sizeof(T) == 8 ? 512 : 1024;
-  if (nx > tmax) return set_error(M3DRT_ELIMIT, "m3drt_sc_sweep: nx beyond the workgroup size");
   const int smax = std::max(1, tmax / nx);
   int L = (ny + smax - 1) / smax;
-  if (L > 32) return set_error(M3DRT_ELIMIT, "m3drt_sc_sweep: ny too large for the strip mapping");
   // the straight-line form when only J (and PsiJ), or only the intensity cube, are
   // asked for and an instantiated strip length divides ny
   int Lexact = 0;
@@ -475,23 +502,13 @@ static int run_sc2(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const m3drt_sweep_
   cc(h1, kx);
   cc(h2, ky);
 
-  // in-plane offsets are 32-bit: every (x, y) offset of a cube and plane must fit
-  const uint64_t span = (uint64_t)(nx - 1) * d->cs_x + (uint64_t)(ny - 1) * d->cs_y;
-  const uint64_t gspan = (uint64_t)(nx - 1) * d->gs_x + (uint64_t)(ny - 1) * d->gs_y;
-  if ((span + 1) * sizeof(T) >= (1ull << 32) || (gspan + 1) * sizeof(T) >= (1ull << 32))
-    return set_error(M3DRT_ELIMIT, "m3drt_sc_sweep: in-plane offsets exceed 32 bits");
-
   const size_t nprep = (size_t)nxy * (nz + 1);
   int rc = ensure_scratch(ctx, sizeof(T) * 2 * nprep);
   if (rc) return rc;
   T *dt500 = static_cast<T *>(ctx->scratch);
   T *rcp = dt500 + nprep;
-  {
-    const int blocks = (int)std::min<int64_t>(((int64_t)nprep + 255) / 256, 65536);
-    hipLaunchKernelGGL(sc2_prep<T>, dim3(blocks), dim3(256), 0, ctx->stream, b->chi500, b->chi500_up,
-                       b->g500, dt500, rcp, (int)nxy, nz, dsup);
-    M3DRT_HIP(hipGetLastError());
-  }
+  rc = sc2_prep<T>(ctx, d, b->chi500, b->chi500_up, b->g500, dt500, rcp);
+  if (rc) return rc;
 
   Sc2Args<T> a;
   a.chi = static_cast<const T *>(b->chi);
@@ -547,11 +564,21 @@ static int run_sc2(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const m3drt_sweep_
   return dispatch_lds<T, 32>(ctx, a, nt, nplanes);
 }
 
+template <typename T>
+static int route_sc2(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const m3drt_sweep_bufs *b) {
+  const int lim = sc2_limits<T>(ctx, d);
+  if (lim) return lim;
+  const int plane = sweep_sc2_plane<T>(ctx, d, b);
+  if (plane >= 0) return plane;
+  if (sizeof(T) == 4) {
+    const int fast = sweep_sc2_fast(ctx, d, b);
+    if (fast >= 0) return fast;
+  }
+  return run_sc2<T>(ctx, d, b);
+}
+
 int sweep_sc2(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const m3drt_sweep_bufs *b) {
-  const int fast = sweep_sc2_fast(ctx, d, b);
-  if (fast >= 0) return fast;
-  if (d->prec == M3DRT_F64) return run_sc2<double>(ctx, d, b);
-  return run_sc2<float>(ctx, d, b);
+  return d->prec == M3DRT_F64 ? route_sc2<double>(ctx, d, b) : route_sc2<float>(ctx, d, b);
 }
 
 }  // namespace m3drt

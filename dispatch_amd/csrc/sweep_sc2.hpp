@@ -38,6 +38,16 @@ inline Sc2Geom sc2_geometry(const m3drt_sweep_desc *d) {
 // the context's scratch: the per-direction preparation of the short_char2 sweeps.
 int sc2_prep_f32(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const float *chi500, const float *chi500_up,
                  const float *g500, float **dt500, float **rc);
+// the same into caller-given arrays of nx*ny*(nz+1) elements each
+template <typename T>
+int sc2_prep(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const float *chi500, const float *chi500_up,
+             const float *g500, T *dt500, T *rc);
+
+// The plane-by-plane sweep of cubes with the frequencies at unit stride; returns -1
+// when the case is not one it takes, else a status.  The caller has made the checks of
+// the general kernel.
+template <typename T>
+int sweep_sc2_plane(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const m3drt_sweep_bufs *b);
 
 // The straight-line sweep for J (and PsiJ) only; returns -1 when the case is not
 // one it takes (the caller then runs the general kernel), else a status.

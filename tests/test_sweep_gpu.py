@@ -406,3 +406,37 @@ def test_sweep_hermite(ctx, kw):
     if split:
         check32(back(Irem), irem, "Irem hermite")
         check32(back(Esc), esc, "escape hermite")
+
+
+# the plane-by-plane form (frequencies at unit stride): waves of 16, 32 and 64
+# frequencies with idle lanes, strips cut short, planes narrower than the stencil, and
+# column groups that do not divide nx, for every strip length.
+@pytest.mark.parametrize("rows,nf,nx,ny,nz,vec", [
+    (1, 16, 3, 2, 4, (0.3, -0.4, 0.866)), (8, 17, 5, 9, 5, (-0.5, 0.2, -0.84)), (4, 32, 9, 8, 3, (0.1, 0.97, 0.211)),
+    (4, 33, 17, 13, 4, (0.61481017, 0.0, 0.78867513)), (2, 64, 1, 7, 3, (0.4, 0.5, -0.7)),
+    (8, 100, 10, 1, 6, (-0.4, 0.5, 0.7)), (8, 130, 6, 17, 1, (0.9, 0.2, 0.39)),
+])
+def test_sweep_plane_form_matches_oracle(ctx, monkeypatch, rows, nf, nx, ny, nz, vec):
+    monkeypatch.setenv("M3DRT_PLANE_ALWAYS", "1")
+    monkeypatch.setenv("M3DRT_PLANE_L", str(rows))
+    case = make_case(nf=nf, nx=nx, ny=ny, nz=nz, seed=nf, vec=vec, maser=nf == 33)
+    print(f"plane form strips of {rows} nf={nf} plane={nx}x{ny} nz={nz}", flush=True)
+    I, psi, irem, esc = run_oracle(case, split_rates=True)
+    J = 0.125 + 0.25 * interior(I).astype(np.float64)
+    g = run_gpu(ctx, case, "reference", split_rates=True)
+    for k, ref in dict(I=interior(I), Psi=psi, Irem=irem, esc=esc, J=J,
+                       PsiJ=0.5 + 0.25 * psi.astype(np.float64)).items():
+        check32(g[k], ref, k)
+    last = case["nz"] if case["dir"] > 0 else 1
+    check32(g["exit"], I[last], "exit plane")
+    I64, psi64, _, _ = run_oracle(case, fp64=True)
+    g = run_gpu(ctx, case, "reference", dtype=torch.float64)
+    assert max_rel(g["I"], interior(I64), 1e-12) < 1e-11
+    # J alone (no rates): the form the formal solution of an iteration takes
+    d = lambda a: dev(a)
+    gz = case["gz"]
+    Jd = torch.full((nz, ny, nx, nf), 0.125, device="cuda")
+    ctx.sc_sweep(d(interior(case["chi"])), d(interior(case["S"])), d(case["chi"][gz]), d(case["S"][gz]),
+                 d(case["I"][gz]), d(case["chi500"]), d(case["chi500_up"]), d(case["g500"]), dir=case["dir"],
+                 ds=case["ds"], vec=case["vec"], layout="reference", wj=0.25, J=Jd)
+    check32(Jd.cpu().numpy(), 0.125 + 0.25 * interior(run_oracle(case)[0]).astype(np.float64), "J alone")
