@@ -34,6 +34,7 @@ namespace m3drt {
 namespace {
 
 constexpr int QLG_NX = 9019;
+constexpr int kOpacThreads = 256;
 
 struct OpacArgs {
   int nline;
@@ -206,12 +207,15 @@ __global__ void __launch_bounds__(1024) select_lines_kernel(const double *__rest
   if (tid == 0) sel[0] = base;
 }
 
-// qlg_bot_line_eval (HOP/qlg_mod.f90:542-556) at abscissa x
+// qlg_bot_line_eval (HOP/qlg_mod.f90:542-556) at abscissa x.  The table index is the
+// nearest integer, halves upwards: for 0 <= v < 2^23 exactly the integer part of
+// v + (0.5 - 2^-25), an addition and a conversion where roundf takes seven operations
+// (adding 0.5 itself would round the largest float below 0.5 up to 1).
 __device__ __forceinline__ float bot_eval(const Coef &c, float x, const float *TGX, const float *TH2X) {
   const float xs = fabsf(x) * c.ih;
   const float u = xs * xs;
   const float L = __builtin_amdgcn_rcpf(1.0f + u);
-  const int ig = nint(fminf(xs * 800.0f, (float)QLG_NX));
+  const int ig = (int)(fminf(xs * 800.0f, (float)QLG_NX) + 0.49999997f);
   const float G = TGX[ig], W = TH2X[ig];
   float p = c.cL2 + c.cZH * W;
   p = c.bL + L * p;
@@ -227,7 +231,7 @@ __device__ __forceinline__ float bot_eval(const Coef &c, float x, const float *T
 // time, and the scattering path leaves the per-point code.  The direct form never
 // takes the split.
 template <bool GENERAL, bool DIRECT, bool SCAT>
-__global__ void __launch_bounds__(256) opacity_kernel(const OpacArgs a) {
+__global__ void __launch_bounds__(kOpacThreads) opacity_kernel(const OpacArgs a) {
   static_assert(!(DIRECT && SCAT), "the direct form takes no scattering split");
   extern __shared__ float tab[];  // TGX then TH2X
   for (int i = threadIdx.x; i <= QLG_NX; i += blockDim.x) {
@@ -236,8 +240,12 @@ __global__ void __launch_bounds__(256) opacity_kernel(const OpacArgs a) {
   }
   __syncthreads();
   const float *TGX = tab, *TH2X = tab + QLG_NX + 1;
-  const int cidx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (cidx >= a.ncell) return;
+  // lanes beyond the last cell walk along with it (the deposits are taken by whole
+  // waves) but never queue a line, so they read and write nothing of the spectra
+  const int cell = blockIdx.x * blockDim.x + threadIdx.x;
+  const bool alive = cell < a.ncell;
+  if (!__any(alive)) return;
+  const int cidx = min(cell, a.ncell - 1);
 
   const float sqrt_pi = 1.7724538509f, ex_cutoff = -85.0f, voigt_peak = 0.5641895835f;
   const int nf = a.nf;
@@ -269,16 +277,19 @@ __global__ void __launch_bounds__(256) opacity_kernel(const OpacArgs a) {
   // needs chi at its centre node as the sequential order has it there: the global
   // value (every earlier chunk deposited) plus the pending lines' deposits at that
   // node, added in line order with the same FP32 operations.
-  constexpr int K = 4;
+  constexpr int K = 4, U = SCAT ? 4 : 8;
   Pend pend[K];
   int np = 0, fc = 1;
   const double *llam = a.llam;
   auto val = [&](const Pend &q, int f) -> float {
-    const float x = GENERAL ? (float)(llam[f - 1] - q.llc) : q.x0 + (float)(f - q.fa);
+    const float x = GENERAL ? (float)(dev::ro(llam)[f - 1] - q.llc) : q.x0 + (float)(f - q.fa);
     return bot_eval(q.c, x, TGX, TH2X);
   };
+  // The deposit walks the frequencies of the wave's windows together, so that at every
+  // frequency the lanes that take part access one contiguous run of cells: neighbouring
+  // cells' windows are shifted by their velocities, and lanes walking each its own
+  // window would each access another row of the spectrum.
   auto flush = [&]() {
-    if (np == 0) return;
     int Fa = nf + 1, Fb = 0;
     bool anyscat = false;
 #pragma unroll
@@ -287,15 +298,25 @@ __global__ void __launch_bounds__(256) opacity_kernel(const OpacArgs a) {
         Fa = min(Fa, pend[k].fa);
         Fb = max(Fb, pend[k].fb);
         anyscat = anyscat || !(!SCAT || pend[k].plain);
+      } else {
+        pend[k].fa = nf + 1;  // no point's window
+        pend[k].fb = 0;
       }
     }
-    constexpr int U = 8;
+#pragma unroll
+    for (int m = 1; m < 64; m *= 2) {
+      Fa = min(Fa, __shfl_xor(Fa, m));
+      Fb = max(Fb, __shfl_xor(Fb, m));
+    }
+    Fa = __builtin_amdgcn_readfirstlane(Fa);
+    Fb = __builtin_amdgcn_readfirstlane(Fb);
+    if (SCAT) anyscat = __any(anyscat);
     for (int f = Fa; f <= Fb; f += U) {
       bool any = false;
 #pragma unroll
-      for (int k = 0; k < K; ++k) any = any || (k < np && pend[k].fa <= f + U - 1 && pend[k].fb >= f);
+      for (int k = 0; k < K; ++k) any = any || (pend[k].fa <= f + U - 1 && pend[k].fb >= f);
       if (!any) continue;
-      float cv[U], ev[U], sv[U], ov[U], cb[DIRECT ? U : 1], eb[DIRECT ? U : 1];
+      float cv[U], ev[U], sv[SCAT ? U : 1], ov[SCAT ? U : 1], cb[DIRECT ? U : 1], eb[DIRECT ? U : 1];
 #pragma unroll
       for (int j = 0; j < U; ++j) {
         if (f + j <= Fb) {
@@ -309,7 +330,7 @@ __global__ void __launch_bounds__(256) opacity_kernel(const OpacArgs a) {
             cv[j] = chi[o];
             ev[j] = eta[o];
           }
-          if (anyscat) {
+          if (SCAT && anyscat) {
             sv[j] = csc_c[o];
             ov[j] = ome_c[o];
           }
@@ -317,21 +338,20 @@ __global__ void __launch_bounds__(256) opacity_kernel(const OpacArgs a) {
       }
 #pragma unroll
       for (int k = 0; k < K; ++k) {
-        if (k < np) {
+        const int fa = pend[k].fa, fb = pend[k].fb;
+        if (fa <= f + U - 1 && fb >= f) {
+          const bool plain = !SCAT || pend[k].plain;
 #pragma unroll
           for (int j = 0; j < U; ++j) {
             const int g = f + j;
-            if (g >= pend[k].fa && g <= pend[k].fb) {
-              const float lte = val(pend[k], g);
-              if (!SCAT || pend[k].plain) {
-                cv[j] = cv[j] + lte * pend[k].bi;
-                ev[j] = ev[j] + lte * pend[k].bj;
-              } else {
-                cv[j] = cv[j] + lte;
-                ev[j] = ev[j] + lte;
-                sv[j] = sv[j] + ov[j] * lte;
-              }
-            }
+            if (GENERAL && g > nf) break;  // its node is beyond the grid
+            const float lte = val(pend[k], g);
+            // a point outside the window keeps its sums
+            const bool in = g >= fa && g <= fb;
+            const float dc = plain ? lte * pend[k].bi : lte, de = plain ? lte * pend[k].bj : lte;
+            cv[j] = in ? cv[j] + dc : cv[j];
+            ev[j] = in ? ev[j] + de : ev[j];
+            if (SCAT) sv[j] = in && !plain ? sv[j] + ov[j] * lte : sv[j];
           }
         }
       }
@@ -346,7 +366,7 @@ __global__ void __launch_bounds__(256) opacity_kernel(const OpacArgs a) {
             chi[o] = cv[j];
             eta[o] = ev[j];
           }
-          if (anyscat) csc_c[o] = sv[j];
+          if (SCAT && anyscat) csc_c[o] = sv[j];
         }
       }
     }
@@ -356,7 +376,7 @@ __global__ void __launch_bounds__(256) opacity_kernel(const OpacArgs a) {
 #pragma unroll
     for (int k = 0; k < K; ++k)
       if (k == np) pend[k] = q;
-    if (++np == K) flush();
+    ++np;
   };
 
   auto lref_at = [&](int f) -> float {
@@ -365,8 +385,8 @@ __global__ void __launch_bounds__(256) opacity_kernel(const OpacArgs a) {
     return x > 0.0f ? a.lt + (float)log((double)x) : -3.40282347e38f;
   };
   const int nsel = a.sel ? a.sel[0] : a.nline;
-  for (int is = 0; is < nsel; ++is) {
-    const int l = a.sel ? a.sel[1 + is] : is;
+  // one line: its decision, and its place among the pending lines if it passes
+  auto consider = [&](int l) {
     const double llc = a.llam0[l] - (double)vproj_c;
     const double pos = (llc - llam1) * inv_dllam;
     int f0;
@@ -381,7 +401,7 @@ __global__ void __launch_bounds__(256) opacity_kernel(const OpacArgs a) {
     const float ex = a.lower_ev[l] * ekt;
     const int ip = a.ipart ? a.ipart[l] : 1;
     const float arg = a.lnbase[(int64_t)(ip - 1) * a.ncell + cidx] + a.gpref[l] - ex;
-    if (arg < ex_cutoff) continue;
+    if (arg < ex_cutoff) return;
     // a line centred beyond the grid, in a list with reaches: the reference is the
     // continuum at the nearer grid end, without the running floor (:594-602, 844-851)
     const bool outside = a.reach_in && (llc < a.llam[0] || llc > a.llam[nf - 1]);
@@ -389,7 +409,7 @@ __global__ void __launch_bounds__(256) opacity_kernel(const OpacArgs a) {
     if (outside) {
       const int fe = llc < a.llam[0] ? 1 : nf;
       const float lref_o = lref_at(fe);
-      if (arg <= lref_o) continue;
+      if (arg <= lref_o) return;
       Rij = (float)exp((double)arg);
       ref = a.tol * cont[(fe - 1) * sf];
       lnq = arg - lref_o;
@@ -413,10 +433,10 @@ __global__ void __launch_bounds__(256) opacity_kernel(const OpacArgs a) {
       } else {
         lref_c = lref_at(f0);
       }
-      if (arg <= lref_c) continue;
+      if (arg <= lref_c) return;
       Rij = (float)exp((double)arg);
       ref = refl_c;
-      if (voigt_peak * Rij <= ref) continue;
+      if (voigt_peak * Rij <= ref) return;
       lnq = arg - lref_c;
     }
 
@@ -462,7 +482,7 @@ __global__ void __launch_bounds__(256) opacity_kernel(const OpacArgs a) {
           hb0 = 0.5 * (a.llam[1] - a.llam[0]);
           hb1 = 0.5 * (a.llam[nf - 1] - a.llam[nf - 2]);
         }
-        if (llc + dl < a.llam[0] - hb0 || llc - dl > a.llam[nf - 1] + hb1) continue;
+        if (llc + dl < a.llam[0] - hb0 || llc - dl > a.llam[nf - 1] + hb1) return;
         if (a.used) a.used[l] = 1;
         q.fa = bisect_nearest(a.llam, 1, nf, llc - dl);
         q.fb = bisect_nearest(a.llam, 1, nf, llc + dl);
@@ -475,9 +495,9 @@ __global__ void __launch_bounds__(256) opacity_kernel(const OpacArgs a) {
           q.fb = bisect_nearest(a.llam, f0, nf, llc + dl);
         }
       }
-      if (q.fa > q.fb) continue;
+      if (q.fa > q.fb) return;
       queue(q);
-      continue;
+      return;
     }
 
     // qlg_bot_line_sweep (HOP/qlg_mod.f90:630-653): setup, window, sweep
@@ -495,12 +515,16 @@ __global__ void __launch_bounds__(256) opacity_kernel(const OpacArgs a) {
     const int noff = nint(fminf(fminf(hw, cap), (float)(nf + abs(ic))));
     q.fa = max(1, ic - noff);
     q.fb = min(nf, ic + noff);
-    if (q.fa > q.fb) continue;
+    if (q.fa > q.fb) return;
     if (a.used) a.used[l] = 1;
     q.x0 = x1 - (float)(i1 - q.fa);
     queue(q);
+  };
+  for (int is = 0; is < nsel; ++is) {
+    if (alive) consider(a.sel ? a.sel[1 + is] : is);
+    if (__any(np == K)) flush();
   }
-  flush();
+  if (__any(np > 0)) flush();
 }
 
 // ------------------------------------------------------------------ tables
@@ -614,7 +638,7 @@ int line_opacity(m3drt_ctx *ctx, const m3drt_linelist *ll, const m3drt_opacity_a
   a.lt = (float)log((double)(o->tolerance / 0.5641895835f));
   a.tgx = ctx->qlg_tab;
   a.th2x = ctx->qlg_tab + QLG_NX + 1;
-  const int threads = 256;
+  const int threads = kOpacThreads;
   const int blocks = (o->ncell + threads - 1) / threads;
   const size_t lds = 2 * (QLG_NX + 1) * sizeof(float);
   auto kern = direct ? (general ? opacity_kernel<true, true, false> : opacity_kernel<false, true, false>)
