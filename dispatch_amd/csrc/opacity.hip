@@ -277,7 +277,7 @@ __global__ void __launch_bounds__(kOpacThreads) opacity_kernel(const OpacArgs a)
   // needs chi at its centre node as the sequential order has it there: the global
   // value (every earlier chunk deposited) plus the pending lines' deposits at that
   // node, added in line order with the same FP32 operations.
-  constexpr int K = 4, U = SCAT ? 4 : 8;
+  constexpr int K = DIRECT ? 4 : 12, U = 8;
   Pend pend[K];
   int np = 0, fc = 1;
   const double *llam = a.llam;
