@@ -374,8 +374,11 @@ class NlteProblem:
         f32 = lambda: torch.empty((nf, nc), dtype=torch.float32, device=self.device)
         i32 = lambda: torch.empty((nf, nc), dtype=torch.int32, device=self.device)
         xhat, ehat = f32(), f32()
-        sp = dict(split_opac1=f32(), split_opac2=f32(), split_chi1=f32(), split_chi2=f32(), split_id=i32(),
-                  split_chi_id=i32())
+        # the fused pass leaves the tracking to the rates, which form it again from the
+        # continuum (a context without that call takes the arrays)
+        retrack = self.cfg.fused and self.cfg.precond and hasattr(ctx, "bb_rates_window")
+        sp = {} if retrack else dict(split_opac1=f32(), split_opac2=f32(), split_chi1=f32(), split_chi2=f32(),
+                                     split_id=i32(), split_chi_id=i32())
         I, Psi, Irem, esc = f32(), f32(), f32(), f32()
         sweep64 = self.sweep_dtype == torch.float64
         l0, l1 = w.lines[0], w.lines[-1] + 1
@@ -384,7 +387,9 @@ class NlteProblem:
         for r, v in enumerate(self.vec):
             vproj = (self.vz * (v[2] / CC)).float().contiguous()
             d = dict(w.const, vproj=vproj, **cells)
-            if self.cfg.fused:
+            if retrack:
+                ctx.window_opacity(d, w.chi_c, w.Bnu, w.beta, xhat, ehat, track=True)
+            elif self.cfg.fused:
                 # the same steps as below in one kernel (m3drt_window_opacity)
                 ctx.window_opacity(d, w.chi_c, w.Bnu, w.beta, xhat, ehat, split=sp, split_offset=0)
             else:
@@ -411,9 +416,14 @@ class NlteProblem:
             else:
                 self._sweep(r, chi, S, w.ghost_B, I_out=I, Psi_out=Psi, Irem_out=Irem, escape_out=esc,
                             split_rates=True, get_rates=True)
-            ctx.bb_rates(dict(d, Inu=I, Psi=Psi, Bnu=w.Bnu, beta=w.beta), float(self.wj[r]), 1.0,
-                         gij[l0:l1], gji[l0:l1], precond=self.cfg.precond, own_norm=True, largest=True,
-                         split=dict(sp, Irem=Irem, escape=esc, chi=chi), split_offset=0)
+            dr = dict(d, Inu=I, Psi=Psi, Bnu=w.Bnu, beta=w.beta)
+            parts = dict(sp, Irem=Irem, escape=esc, chi=chi)
+            if retrack:
+                ctx.bb_rates_window(dr, w.chi_c, float(self.wj[r]), 1.0, gij[l0:l1], gji[l0:l1], own_norm=True,
+                                    split=parts, split_offset=0)
+            else:
+                ctx.bb_rates(dr, float(self.wj[r]), 1.0, gij[l0:l1], gji[l0:l1], precond=self.cfg.precond,
+                             own_norm=True, largest=True, split=parts, split_offset=0)
 
     def rates(self):
         """The radiative rate sums of one iteration: (gamma_ij, gamma_ji), (nrad, ncell)

@@ -385,35 +385,49 @@ int m3drt_normalize_rates(m3drt_ctx *ctx, const m3drt_rate_solve_args *r, const 
   return m3drt::normalize_rates(ctx, r, wphi);
 }
 
-int m3drt_bb_rates(m3drt_ctx *ctx, const m3drt_bb_rates_args *r) {
-  if (!ctx || !r) return set_error(M3DRT_EINVAL, "m3drt_bb_rates: NULL argument");
+static int bb_rates_entry(m3drt_ctx *ctx, const m3drt_bb_rates_args *r, const float *cont, bool window) {
+  const std::string w = window ? "m3drt_bb_rates_window: " : "m3drt_bb_rates: ";
+  if (!ctx || !r) return set_error(M3DRT_EINVAL, w + "NULL argument");
   if (r->nline < 0 || r->nf < 0 || r->ncell < 0 || r->nk < 1)
-    return set_error(M3DRT_EINVAL, "m3drt_bb_rates: inconsistent sizes");
+    return set_error(M3DRT_EINVAL, w + "inconsistent sizes");
   if (r->nline == 0 || r->ncell == 0) return M3DRT_OK;
   if (!r->iblue || !r->ired || !r->lev_i || !r->lev_j || !r->Aij || !r->lower_off || !r->q || !r->wnu ||
       !r->g || !r->b || !r->nstar || !r->inv_df || !r->vproj || !r->e_kT || !r->adamp || !r->Inu ||
       !r->Bnu || !r->gamma_ij || !r->gamma_ji)
-    return set_error(M3DRT_EINVAL, "m3drt_bb_rates: missing array");
+    return set_error(M3DRT_EINVAL, w + "missing array");
+  if (window && !cont) return set_error(M3DRT_EINVAL, w + "missing chi_cont");
   const bool precond = r->flags & M3DRT_RATES_PRECOND, largest = r->flags & M3DRT_RATES_LARGEST;
   if (precond && (!r->beta || !r->Bij || !r->pop_ratio))
-    return set_error(M3DRT_EINVAL, "m3drt_bb_rates: preconditioning needs beta, Bij, pop_ratio");
+    return set_error(M3DRT_EINVAL, w + "preconditioning needs beta, Bij, pop_ratio");
   if (precond && !largest && !r->Psi)
-    return set_error(M3DRT_EINVAL, "m3drt_bb_rates: preconditioning needs Psi");
-  if (precond && largest &&
+    return set_error(M3DRT_EINVAL, w + "preconditioning needs Psi");
+  if (window && !(precond && largest))
+    return set_error(M3DRT_EINVAL, w + "'largest' with preconditioning only");
+  if (window && (!r->Psi || !r->Irem || !r->escape || !r->chi))
+    return set_error(M3DRT_EINVAL, w + "Psi, Irem, escape and chi are needed");
+  if (!window && precond && largest &&
       (!r->Psi || !r->Irem || !r->escape || !r->chi || !r->split_opac1 || !r->split_opac2 ||
        !r->split_chi1 || !r->split_chi2 || !r->split_id || !r->split_chi_id))
     return set_error(M3DRT_EINVAL,
-                     "m3drt_bb_rates: 'largest' with preconditioning needs Psi, Irem, escape, chi and the "
+                     w + "'largest' with preconditioning needs Psi, Irem, escape, chi and the "
                      "tracked contributions");
   if ((r->flags & M3DRT_RATES_SCAT) && (!r->chi_scat || !r->dJnu))
-    return set_error(M3DRT_EINVAL, "m3drt_bb_rates: line scattering needs chi_scat and dJnu");
+    return set_error(M3DRT_EINVAL, w + "line scattering needs chi_scat and dJnu");
   if ((r->flags & M3DRT_RATES_FLAGS) && (!r->ntrans || !r->psi_flags_in || !r->psi_flags_out || r->npw < 1))
-    return set_error(M3DRT_EINVAL, "m3drt_bb_rates: psi flags need ntrans, psi_flags_in/out and npw");
+    return set_error(M3DRT_EINVAL, w + "psi flags need ntrans, psi_flags_in/out and npw");
   if ((r->flags & M3DRT_RATES_OWN_NORM) && !r->wq)
-    return set_error(M3DRT_EINVAL, "m3drt_bb_rates: own normalisation needs wq");
-  if (r->sf < 1 || r->sc < 1) return set_error(M3DRT_EINVAL, "m3drt_bb_rates: strides must be >= 1");
+    return set_error(M3DRT_EINVAL, w + "own normalisation needs wq");
+  if (r->sf < 1 || r->sc < 1) return set_error(M3DRT_EINVAL, w + "strides must be >= 1");
   M3DRT_HIP(hipSetDevice(ctx->device));
-  return m3drt::bb_rates(ctx, r);
+  return m3drt::bb_rates(ctx, r, cont);
+}
+
+int m3drt_bb_rates(m3drt_ctx *ctx, const m3drt_bb_rates_args *r) {
+  return bb_rates_entry(ctx, r, nullptr, false);
+}
+
+int m3drt_bb_rates_window(m3drt_ctx *ctx, const m3drt_bb_rates_args *r, const float *chi_cont) {
+  return bb_rates_entry(ctx, r, chi_cont, true);
 }
 
 int m3drt_bb_opacity(m3drt_ctx *ctx, const m3drt_bb_opacity_args *r) {

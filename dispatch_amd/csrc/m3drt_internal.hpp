@@ -57,7 +57,8 @@ int line_opacity(m3drt_ctx *ctx, const m3drt_linelist *ll, const m3drt_opacity_a
                  bool lref_from_cont = false, bool direct = false);
 int rate_solve(m3drt_ctx *ctx, const m3drt_rate_solve_args *r, m3drt_rate_solve_result *res);
 int normalize_rates(m3drt_ctx *ctx, const m3drt_rate_solve_args *r, const float *wphi);
-int bb_rates(m3drt_ctx *ctx, const m3drt_bb_rates_args *r);
+// chi_cont: the tracked contributions formed again from it (m3drt_bb_rates_window); NULL: read
+int bb_rates(m3drt_ctx *ctx, const m3drt_bb_rates_args *r, const float *chi_cont = nullptr);
 int sweep_lcq(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const m3drt_sweep_bufs *b);
 int sweep_lcl(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const m3drt_sweep_bufs *b);
 int sweep_sc1(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const m3drt_sweep_bufs *b);

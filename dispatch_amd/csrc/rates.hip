@@ -28,6 +28,14 @@ namespace {
 
 constexpr int QLG_NX = 9019;
 
+// Threads of the rate and window kernels.  The profile tables take 72 KB of LDS, so two
+// workgroups run on a CU whatever their size; with 256 threads those are two waves a
+// SIMD, too few to hide the loads of these streaming loops.  On the 432 000-cell window
+// of 2400 frequencies: rates 9.8 ms with 384 threads, 6.8 with 512, 8.0 with 640 and 7.1
+// with 768 (one workgroup a CU at this register use); window opacity 5.4 with 512, 4.4
+// with 768, 5.8 with 896 (one workgroup a CU) and 5.3 with 1024 (spills).
+constexpr int kRateThreads = 512, kWinThreads = 768;
+
 struct Kahan {
   float s = 0.0f, c = 0.0f;
   __device__ __forceinline__ void add(float v) {
@@ -56,7 +64,8 @@ struct Qlg {
                                            float idf) const {
     const float v = fabsf(qf - vpr) * idf;
     const float xs = v * ih, u = xs * xs, L = 1.0f / (1.0f + u);
-    const int ig = (int)roundf(fminf(xs * 800.0f, (float)QLG_NX));
+    // the nearest integer, halves upwards: exact for 0 <= v < 2^23 (opacity.hip)
+    const int ig = (int)(fminf(xs * 800.0f, (float)QLG_NX) + 0.49999997f);
     float p = cL2 + cZH * TH2X[ig];
     p = bL + L * p;
     const float K = TGX[ig] * gG + L * p;
@@ -75,6 +84,19 @@ __device__ __forceinline__ float other_contribution(float value, int index, floa
   return index == largest_index ? rest : largest + (rest - value);
 }
 
+// add_largest, SRC/rt_patch_mod.f90:3150-3169
+__device__ __forceinline__ void add_largest(float value, int index, float *largest, float *rest,
+                                            int32_t *largest_index) {
+  const float lg = *largest;
+  if (fabsf(value) > fabsf(lg)) {
+    *rest = *rest + lg;
+    *largest = value;
+    *largest_index = index;
+  } else {
+    *rest = *rest + value;
+  }
+}
+
 // ---------------------------------------------------------------- line rates
 
 struct RatesArgs {
@@ -84,6 +106,7 @@ struct RatesArgs {
   const float *lower_off, *q, *inv_df, *vproj, *e_kT, *adamp;
   const float *Inu, *Psi, *Bnu, *beta;
   const float *Irem, *esc, *chi, *so1, *so2, *sc1, *sc2, *chi_scat, *dJnu;
+  const float *cont;  // the continuum opacity the tracking is formed from again (RETRACK)
   const int32_t *sid, *scid, *ntrans, *flags_in;
   int32_t *flags_out;
   int64_t sf, sc;
@@ -97,7 +120,16 @@ struct RatesArgs {
 // consecutive cells; each run's cells padded to whole workgroups, so k is the
 // workgroup's (the line parameters stay scalar loads).  Each line's sums are its own
 // (one lane per (line, cell)), so the runs change no result.
-__global__ void __launch_bounds__(256) bb_rates_kernel(const RatesArgs a) {
+//
+// RETRACK ('largest' with preconditioning): the tracked contributions of a point are
+// formed again from the continuum and the lines covering it, with window_cell's
+// operations in its order, instead of read.  A line's own profile is at hand here and
+// windows mostly hold one line at a frequency, so this replaces 24 B a point, written
+// by the opacity pass and read here, by the 4 B of the continuum.  On the 432 000-cell
+// window of 2400 frequencies, with the threads above: opacity 12.8 -> 4.4 ms (20 B a
+// point, 4.7 TB/s), rates 9.9 -> 6.8 ms (32 B a point, 4.9 TB/s: HBM-bound).
+template <bool RETRACK, typename O>
+__global__ void __launch_bounds__(kRateThreads) bb_rates_kernel(const RatesArgs a) {
   extern __shared__ float tab[];
   load_tables(tab, a.tab);
   const float *TGX = tab, *TH2X = tab + QLG_NX + 1;
@@ -107,13 +139,14 @@ __global__ void __launch_bounds__(256) bb_rates_kernel(const RatesArgs a) {
   const int nc = a.ncell;
   const bool split_pre = a.largest && a.precond;
   const float idf = a.inv_df[c], vpr = a.vproj[c], ekt = a.e_kT[c];
+  O co = (O)c * (O)a.sc;  // the cell's offset, at a frequency's wave-uniform base
   const int l_hi = min(a.nline, (k + 1) * a.lchunk);
   for (int l = k * a.lchunk; l < l_hi; ++l) {
     // a window or a level outside the arrays skips the line (documented in the header)
-    const int fs = max(a.iblue[l] - 1, 0), fe = min(a.ired[l] - 1, a.nf - 1);
-    const int li = a.lev_i[l] - 1, lj = a.lev_j[l] - 1;
+    const int fs = max(dev::ro(a.iblue)[l] - 1, 0), fe = min(dev::ro(a.ired)[l] - 1, a.nf - 1);
+    const int li = dev::ro(a.lev_i)[l] - 1, lj = dev::ro(a.lev_j)[l] - 1;
     if (li < 0 || li >= a.nk || lj < 0 || lj >= a.nk) continue;
-    const float lower_off = a.lower_off[l];
+    const float lower_off = dev::ro(a.lower_off)[l];
     const int index = a.split_offset + l + 1;
     const double nsi = a.nstar[(int64_t)li * nc + c], nsj = a.nstar[(int64_t)lj * nc + c];
     float ni = (float)(a.b[(int64_t)li * nc + c] * nsi);
@@ -143,7 +176,7 @@ __global__ void __launch_bounds__(256) bb_rates_kernel(const RatesArgs a) {
     const Qlg Q(a.adamp[(int64_t)l * nc + c]);
     Kahan sA, sI, sP, sw;
     const int64_t lo = (int64_t)l * a.nf;
-    if (split_pre) {
+    if ((RETRACK || split_pre) && fs <= fe) {
       bool in_force = false, raise = false;
       int pw = 0, pb = 0;
       if (a.use_flags) {
@@ -151,21 +184,116 @@ __global__ void __launch_bounds__(256) bb_rates_kernel(const RatesArgs a) {
         pb = (a.ntrans[l] - 1) % 32;
         in_force = (a.flags_in[(int64_t)pw * nc + c] >> pb) & 1;
       }
+      // the other lines at a point, of 64 at a time: masks as in window_cell
+      const bool masked = a.nline <= 64;
+      uint64_t cover = 0;
+      int f_next = fs;
+      auto covers = [&](int m, int f) {
+        const int ms = max(dev::ro(a.iblue)[m] - 1, 0), me = min(dev::ro(a.ired)[m] - 1, a.nf - 1);
+        const int mi = dev::ro(a.lev_i)[m] - 1, mj = dev::ro(a.lev_j)[m] - 1;
+        return f >= ms && f <= me && mi >= 0 && mi < a.nk && mj >= 0 && mj < a.nk;
+      };
+      // every read of a point together and unconditionally (reads under the psi == 0
+      // choice would wait for Psi's), one point ahead of the one summed; the
+      // frequency's own values through the scalar cache
+      struct Point {
+        float psi, bt, I, Ir, es, chi, nb, cont;
+      };
+      auto fetch = [&](int f) -> Point {
+        // opaque, as in window_cell
+        asm volatile("" : "+v"(co));
+        const int64_t fo = (int64_t)f * a.sf;
+        Point p;
+        p.psi = (a.Psi + fo)[co];
+        p.bt = (a.beta + fo)[co];
+        p.I = (a.Inu + fo)[co];
+        p.Ir = (a.Irem + fo)[co];
+        p.es = (a.esc + fo)[co];
+        p.chi = (a.chi + fo)[co];
+        p.nb = (a.Bnu + fo)[co];
+        p.cont = RETRACK ? (a.cont + fo)[co] : 0.0f;
+        return p;
+      };
+      Point pt = fetch(fs);
       for (int f = fs; f <= fe; ++f) {
-        // every read of the point first, unconditionally, so that they are in flight
-        // together (reads under the psi == 0 choice would wait for Psi's); the
-        // frequency's own values through the scalar cache
         const float qf = dev::ro(a.q)[lo + f];
         const double wnu = dev::ro(a.wnu)[lo + f];
         const double wqf = a.own_norm ? dev::ro(a.wq)[lo + f] : 0.0;
-        const int64_t o = (int64_t)f * a.sf + (int64_t)c * a.sc;
-        float psi = a.Psi[o];
-        const float bt = a.beta[o], Iv = a.Inu[o], Ir = a.Irem[o], es = a.esc[o], chv = a.chi[o], nb = a.Bnu[o];
-        const float s1 = a.so1[o], s2 = a.so2[o], c1 = a.sc1[o], c2 = a.sc2[o];
-        const int32_t si = a.sid[o], ci = a.scid[o];
-        const float sct = a.scat ? a.chi_scat[o] * a.dJnu[o] : 0.0f;
+        float psi = pt.psi;
+        const float bt = pt.bt, Iv = pt.I, Ir = pt.Ir, es = pt.es, chv = pt.chi, nb = pt.nb;
+        float s1, s2, c1, c2;
+        int32_t si, ci;
+        if (RETRACK) {
+          // the continuum as contribution 0 (convert_to_work_units)
+          const float e0 = pt.cont * nb;
+          c1 = pt.cont + e0;
+          s1 = e0 / bt;
+          s2 = c2 = 0.0f;
+          si = ci = 0;
+        } else {
+          const int64_t fo = (int64_t)f * a.sf;
+          s1 = (a.so1 + fo)[co];
+          s2 = (a.so2 + fo)[co];
+          c1 = (a.sc1 + fo)[co];
+          c2 = (a.sc2 + fo)[co];
+          si = (a.sid + fo)[co];
+          ci = (a.scid + fo)[co];
+        }
+        const float sct = a.scat ? (a.chi_scat + (int64_t)f * a.sf)[co] * (a.dJnu + (int64_t)f * a.sf)[co] : 0.0f;
+        pt = fetch(min(f + 1, fe));
         const float vph = Q.profile(TGX, TH2X, qf, vpr, idf);
         const float eta_u = vph * eta_coef;
+        if (RETRACK) {
+          auto track = [&](float ev, float cv, int id) {
+            add_largest(ev, id, &s1, &s2, &si);
+            add_largest(cv, id, &c1, &c2, &ci);
+          };
+          // another line at this frequency, its factors formed anew
+          auto track_other = [&](int m) {
+            const int mi = dev::ro(a.lev_i)[m] - 1, mj = dev::ro(a.lev_j)[m] - 1;
+            const float off = dev::ro(a.lower_off)[m];
+            const float mn = (float)(a.nstar[(int64_t)mi * nc + c] * a.pop_ratio[c]);
+            float bi = (float)a.b[(int64_t)mi * nc + c], bj = (float)a.b[(int64_t)mj * nc + c];
+            if (off != 0) {
+              const float eo = (float)exp((double)(-off * ekt));
+              bi = bi * eo;
+              bj = bj * eo;
+            }
+            const float Rij = (float)((double)mn * dev::ro(a.Bij)[m]);
+            const float ph = Qlg(a.adamp[(int64_t)m * nc + c])
+                                 .profile(TGX, TH2X, dev::ro(a.q)[(int64_t)m * a.nf + f], vpr, idf);
+            track(ph * (Rij * bj), ph * (Rij * bi), a.split_offset + m + 1);
+          };
+          if (masked) {
+            if (f >= f_next) {
+              cover = 0;
+              f_next = a.nf;
+              for (int m = 0; m < a.nline; ++m) {
+                const int ms = max(dev::ro(a.iblue)[m] - 1, 0), me = min(dev::ro(a.ired)[m] - 1, a.nf - 1);
+                if (ms > f) {
+                  f_next = min(f_next, ms);
+                } else if (me >= f) {
+                  f_next = min(f_next, me + 1);
+                  if (covers(m, f)) cover |= 1ull << m;
+                }
+              }
+            }
+            if (cover == 1ull << l) {
+              track(eta_u, vph * abs_coef, index);
+            } else {
+              for (uint64_t w = cover; w; w &= w - 1) {
+                const int m = (int)__builtin_ctzll(w);
+                if (m == l) track(eta_u, vph * abs_coef, index);
+                else track_other(m);
+              }
+            }
+          } else {
+            for (int m = 0; m < a.nline; ++m) {
+              if (m == l) track(eta_u, vph * abs_coef, index);
+              else if (covers(m, f)) track_other(m);
+            }
+          }
+        }
         const float eta_t = eta_u * bt;
         const float chi_t = vph * abs_coef - eta_t;
         const float eta_other = bt * other_contribution(eta_u, index, s1, s2, si);
@@ -184,21 +312,21 @@ __global__ void __launch_bounds__(256) bb_rates_kernel(const RatesArgs a) {
         if (a.own_norm) sw.add(vph * (float)wqf);
       }
       if (a.use_flags && raise && !in_force) atomicOr(&a.flags_out[(int64_t)pw * nc + c], (int32_t)(1u << pb));
-    } else {
+    } else if (!RETRACK) {
       for (int f = fs; f <= fe; ++f) {
         const float qf = dev::ro(a.q)[lo + f];
         const float phi = Q.profile(TGX, TH2X, qf, vpr, idf);
         const float wmunu = (float)((double)a.wmu * dev::ro(a.wnu)[lo + f] * a.Aij[l]);
         const float vvv = phi * wmunu;
-        const int64_t o = (int64_t)f * a.sf + (int64_t)c * a.sc;
-        const float nb = a.Bnu[o], Iv = a.Inu[o];
+        const int64_t fo = (int64_t)f * a.sf;
+        const float nb = (a.Bnu + fo)[co], Iv = (a.Inu + fo)[co];
         if (a.own_norm) sw.add(phi * (float)dev::ro(a.wq)[lo + f]);
         sA.add(vvv * (nb * inv_nref));
         if (a.largest) {
           sI.add(vvv * (Iv - nb));
         } else {
           sI.add(vvv * Iv);
-          sP.add(vvv * phi * a.Psi[o] * a.beta[o]);
+          sP.add(vvv * phi * (a.Psi + fo)[co] * (a.beta + fo)[co]);
         }
       }
     }
@@ -233,19 +361,6 @@ struct OpacArgs {
   float wmu;
   const float *tab;
 };
-
-// add_largest, SRC/rt_patch_mod.f90:3150-3169
-__device__ __forceinline__ void add_largest(float value, int index, float *largest, float *rest,
-                                            int32_t *largest_index) {
-  const float lg = *largest;
-  if (fabsf(value) > fabsf(lg)) {
-    *rest = *rest + lg;
-    *largest = value;
-    *largest_index = index;
-  } else {
-    *rest = *rest + value;
-  }
-}
 
 // One line's frequencies of one cell.  The arrays are distinct (restrict): the
 // compiler may then issue the reads of the next frequencies before this one's
@@ -343,7 +458,7 @@ struct WinArgs {
 // contiguous frequency ranges, so a lane re-forms them only where windows overlap).
 // The frequency loop of one cell; the arrays are distinct (restrict), so the reads of
 // the next points need not wait for this point's writes.
-template <bool SPLIT>
+template <bool SPLIT, bool STORE, typename O>
 __device__ __forceinline__ unsigned long long window_cell(
     const OpacArgs &a, const float *TGX, const float *TH2X, int c, int f_lo, int f_hi, float floor_frac, int suppress,
     const float *__restrict__ cont, const float *__restrict__ Bnu, const float *__restrict__ beta,
@@ -404,15 +519,19 @@ __device__ __forceinline__ unsigned long long window_cell(
   // the next point's reads are issued before this point's writes (a deeper ring of
   // four points measured slower: 14.4 against 12.4 ms on the 432 000-cell window, its
   // registers costing a wave per SIMD)
-  int64_t o = (int64_t)c * a.sc + (int64_t)f_lo * a.sf;
-  float cc = cont[o], bn = Bnu[o], bt = beta[o];
+  O co = (O)c * (O)a.sc;  // the cell's offset, at a frequency's wave-uniform base
+  int64_t fo = (int64_t)f_lo * a.sf;
+  float cc = (cont + fo)[co], bn = (Bnu + fo)[co], bt = (beta + fo)[co];
   for (int f = f_lo; f < f_hi; ++f) {
-    const int64_t on = o + a.sf;
+    // opaque, so that the arrays' addresses stay scalar bases plus this offset and are
+    // not summed into a pair of registers each ahead of the loop
+    asm volatile("" : "+v"(co));
+    const int64_t fn = fo + a.sf;
     float ccn = 0.0f, bnn = 0.0f, btn = 0.0f;
     if (f + 1 < f_hi) {
-      ccn = cont[on];
-      bnn = Bnu[on];
-      btn = beta[on];
+      ccn = (cont + fn)[co];
+      bnn = (Bnu + fn)[co];
+      btn = (beta + fn)[co];
     }
     if (masked && f >= f_next) {
       cover = 0;
@@ -455,17 +574,17 @@ __device__ __forceinline__ unsigned long long window_cell(
       chi = copysignf(floor, chi);
       ++floored;
     }
-    xhat[o] = chi;
-    ehat[o] = eta / chi;
-    if (SPLIT) {
-      so1[o] = s1;
-      so2[o] = s2;
-      sidp[o] = sid;
-      sc1[o] = c1;
-      sc2[o] = c2;
-      scidp[o] = cid;
+    (xhat + fo)[co] = chi;
+    (ehat + fo)[co] = eta / chi;
+    if (SPLIT && STORE) {
+      (so1 + fo)[co] = s1;
+      (so2 + fo)[co] = s2;
+      (sidp + fo)[co] = sid;
+      (sc1 + fo)[co] = c1;
+      (sc2 + fo)[co] = c2;
+      (scidp + fo)[co] = cid;
     }
-    o = on;
+    fo = fn;
     cc = ccn;
     bn = bnn;
     bt = btn;
@@ -481,8 +600,11 @@ __device__ __forceinline__ unsigned long long window_cell(
 // (lines in index order at each point) and m3drt_work_to_transfer.  A line's per-cell
 // factors are formed when the frequency loop enters its window (lines cover
 // contiguous frequency ranges, so a lane re-forms them only where windows overlap).
-template <bool SPLIT>
-__global__ void __launch_bounds__(256) window_opacity_kernel(const WinArgs w) {
+// STORE: the tracking arrays are written (else their split only forms eta).
+// O: a cell's offset within one frequency, 32-bit where that holds it (the accesses then
+// take a scalar base and a 32-bit lane offset).
+template <bool SPLIT, bool STORE, typename O>
+__global__ void __launch_bounds__(kWinThreads) window_opacity_kernel(const WinArgs w) {
   extern __shared__ float tab[];
   const OpacArgs &a = w.o;
   load_tables(tab, a.tab);
@@ -496,7 +618,7 @@ __global__ void __launch_bounds__(256) window_opacity_kernel(const WinArgs w) {
   const int f_lo = k * w.fchunk, f_hi = min(a.nf, f_lo + w.fchunk);
   if (f_lo >= f_hi) return;
   const unsigned long long floored =
-      window_cell<SPLIT>(a, TGX, TH2X, c, f_lo, f_hi, w.floor_frac, w.suppress, w.cont, w.Bnu, w.beta, a.xhat,
+      window_cell<SPLIT, STORE, O>(a, TGX, TH2X, c, f_lo, f_hi, w.floor_frac, w.suppress, w.cont, w.Bnu, w.beta, a.xhat,
                          a.ehat, a.so1, a.so2, a.sid, a.sc1, a.sc2, a.scid);
   if (w.n_floored && floored) atomicAdd(w.n_floored, floored);
 }
@@ -551,17 +673,20 @@ __global__ void __launch_bounds__(256) bf_rates_kernel(const BfArgs a) {
   }
 }
 
+// every cell's byte offset within one frequency fits 32 bits (4-byte elements)
+bool offsets32(int64_t ncell, int64_t sc) { return sc < (int64_t)1 << 30 && (ncell - 1) * sc < (int64_t)1 << 30; }
+
 template <typename K, typename A>
-int launch_cells(m3drt_ctx *ctx, K kern, const A &a, int ncell, size_t lds) {
+int launch_cells(m3drt_ctx *ctx, K kern, const A &a, int ncell, size_t lds, int threads = 256) {
   if (lds) M3DRT_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  hipLaunchKernelGGL(kern, dim3((ncell + 255) / 256), dim3(256), lds, ctx->stream, a);
+  hipLaunchKernelGGL(kern, dim3((ncell + threads - 1) / threads), dim3(threads), lds, ctx->stream, a);
   M3DRT_HIP(hipGetLastError());
   return M3DRT_OK;
 }
 
 }  // namespace
 
-int bb_rates(m3drt_ctx *ctx, const m3drt_bb_rates_args *r) {
+int bb_rates(m3drt_ctx *ctx, const m3drt_bb_rates_args *r, const float *chi_cont) {
   int rc = qlg_tables(ctx);
   if (rc) return rc;
   RatesArgs a;
@@ -583,19 +708,23 @@ int bb_rates(m3drt_ctx *ctx, const m3drt_bb_rates_args *r) {
   a.ntrans = r->ntrans; a.flags_in = r->psi_flags_in; a.flags_out = r->psi_flags_out;
   a.sf = r->sf; a.sc = r->sc; a.wmu = r->wmu; a.wtot = r->wtot;
   a.gij = r->gamma_ij; a.gji = r->gamma_ji;
+  a.cont = chi_cont;
   a.tab = ctx->qlg_tab;
   // the lines in runs over enough lanes (about 2M) that the chip holds the grid
-  // several times over (one lane per cell leaves, on the 432 000-cell window, 1688
-  // workgroups against 1280 resident at this kernel's register use)
+  // several times over (one lane per cell leaves, on the 432 000-cell window, 844
+  // workgroups against the 512 the tables' LDS leaves resident)
   const int64_t want = 1 << 21;
   int nchunk = (int)std::max<int64_t>(1, (want + r->ncell - 1) / std::max(1, r->ncell));
   nchunk = std::max(1, std::min(nchunk, r->nline));
   a.lchunk = (r->nline + nchunk - 1) / nchunk;
   a.nchunk = std::max(1, (r->nline + a.lchunk - 1) / std::max(1, a.lchunk));
-  a.ncp = (r->ncell + 255) / 256 * 256;
+  a.ncp = (int)(((int64_t)r->ncell + kRateThreads - 1) / kRateThreads * kRateThreads);
   const int64_t lanes = (int64_t)a.ncp * a.nchunk;
   if (lanes > (int64_t)INT32_MAX) return set_error(M3DRT_ELIMIT, "m3drt_bb_rates: too many points");
-  return launch_cells(ctx, bb_rates_kernel, a, (int)lanes, 2 * (QLG_NX + 1) * sizeof(float));
+  const size_t lds = 2 * (QLG_NX + 1) * sizeof(float);
+  auto run = [&](auto kern) { return launch_cells(ctx, kern, a, (int)lanes, lds, kRateThreads); };
+  if (offsets32(r->ncell, r->sc)) return chi_cont ? run(bb_rates_kernel<true, uint32_t>) : run(bb_rates_kernel<false, uint32_t>);
+  return chi_cont ? run(bb_rates_kernel<true, int64_t>) : run(bb_rates_kernel<false, int64_t>);
 }
 
 int bb_opacity(m3drt_ctx *ctx, const m3drt_bb_opacity_args *r) {
@@ -655,19 +784,27 @@ int window_opacity(m3drt_ctx *ctx, const m3drt_bb_opacity_args *r, const m3drt_w
   const size_t lds = 2 * (QLG_NX + 1) * sizeof(float);
   // Each cell's frequencies in runs of at least 64 over enough lanes (about 2M) that
   // the chip holds the grid several times over: one lane walking all of a cell's
-  // frequencies leaves, on the 432 000-cell window, 1688 workgroups against 1536
-  // resident at this kernel's register use, and the last 152 run a second full-length
-  // round alone.  The points are independent, so the runs change no result.
+  // frequencies leaves, on the 432 000-cell window, 563 workgroups against the 512 the
+  // tables' LDS leaves resident, and the last 51 run a second full-length round alone.
+  // The points are independent, so the runs change no result.
   const int64_t want = 1 << 21;
   int nchunk = (int)std::max<int64_t>(1, (want + r->ncell - 1) / std::max(1, r->ncell));
   nchunk = std::max(1, std::min(nchunk, r->nf / 64));
   w.fchunk = (r->nf + nchunk - 1) / nchunk;
   w.nchunk = (r->nf + w.fchunk - 1) / w.fchunk;
-  w.ncp = (r->ncell + 255) / 256 * 256;
+  w.ncp = (int)(((int64_t)r->ncell + kWinThreads - 1) / kWinThreads * kWinThreads);
   const int64_t lanes = (int64_t)w.ncp * w.nchunk;
   if (lanes > (int64_t)INT32_MAX) return set_error(M3DRT_ELIMIT, "m3drt_window_opacity: too many points");
-  if (a.split) return launch_cells(ctx, window_opacity_kernel<true>, w, (int)lanes, lds);
-  return launch_cells(ctx, window_opacity_kernel<false>, w, (int)lanes, lds);
+  auto run = [&](auto kern) { return launch_cells(ctx, kern, w, (int)lanes, lds, kWinThreads); };
+  const bool track = r->flags & M3DRT_BBOP_TRACK;
+  if (offsets32(r->ncell, r->sc)) {
+    if (track) return run(window_opacity_kernel<true, false, uint32_t>);
+    if (a.split) return run(window_opacity_kernel<true, true, uint32_t>);
+    return run(window_opacity_kernel<false, false, uint32_t>);
+  }
+  if (track) return run(window_opacity_kernel<true, false, int64_t>);
+  if (a.split) return run(window_opacity_kernel<true, true, int64_t>);
+  return run(window_opacity_kernel<false, false, int64_t>);
 }
 
 }  // namespace m3drt

@@ -26,7 +26,7 @@ module m3drt
   integer(c_int), parameter, public :: M3DRT_OPAC_NLTE = 1, M3DRT_OPAC_SCAT = 2
   integer(c_int), parameter, public :: M3DRT_RATES_PRECOND = 1, M3DRT_RATES_OWN_NORM = 2, &
                                        M3DRT_RATES_LARGEST = 4, M3DRT_RATES_SCAT = 8, M3DRT_RATES_FLAGS = 16
-  integer(c_int), parameter, public :: M3DRT_BBOP_LTE = 1, M3DRT_BBOP_SPLIT = 2
+  integer(c_int), parameter, public :: M3DRT_BBOP_LTE = 1, M3DRT_BBOP_SPLIT = 2, M3DRT_BBOP_TRACK = 4
   integer(c_int), parameter, public :: M3DRT_UNITS_SPLIT = 1, M3DRT_UNITS_SCAT = 2, &
                                        M3DRT_UNITS_SUPPRESS_MASERS = 4
   integer(c_int), parameter, public :: M3DRT_BG_SCAT_ALI = 1, M3DRT_BG_J_TO_B = 2
@@ -540,7 +540,7 @@ module m3drt
   public :: m3drt_lc_sweep_hermite, m3drt_lc_sweep_hermite2
   public :: m3drt_sc_sweep_hermite, m3drt_sc_adjoint, m3drt_line_opacity_equi, m3drt_line_opacity
   public :: m3drt_window_opacity, m3drt_rotate_array
-  public :: m3drt_bb_opacity, m3drt_bb_rates, m3drt_bf_rates, m3drt_work_to_transfer
+  public :: m3drt_bb_opacity, m3drt_bb_rates, m3drt_bb_rates_window, m3drt_bf_rates, m3drt_work_to_transfer
   public :: m3drt_convert_to_work_units, m3drt_background_emission, m3drt_update_eta_mask
   public :: m3drt_normalize_rates, m3drt_rate_solve_f64
   public :: m3drt_b1d_synth_plain, m3drt_b1d_plan_create, m3drt_b1d_plan_run, m3drt_b1d_plan_info
@@ -657,6 +657,12 @@ module m3drt
       type(c_ptr), value :: ctx
       type(m3drt_bb_rates_args), intent(in) :: args
     end function m3drt_bb_rates
+    integer(c_int) function m3drt_bb_rates_window(ctx, args, chi_cont) bind(C, name='m3drt_bb_rates_window')
+      import :: c_int, c_ptr, m3drt_bb_rates_args
+      type(c_ptr), value :: ctx
+      type(m3drt_bb_rates_args), intent(in) :: args
+      type(c_ptr), value :: chi_cont
+    end function m3drt_bb_rates_window
     integer(c_int) function m3drt_bf_rates(ctx, args) bind(C, name='m3drt_bf_rates')
       import :: c_int, c_ptr, m3drt_bf_rates_args
       type(c_ptr), value :: ctx

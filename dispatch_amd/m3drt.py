@@ -514,7 +514,7 @@ Context.normalize_rates = _normalize_rates
 
 M3DRT_RATES_PRECOND, M3DRT_RATES_OWN_NORM, M3DRT_RATES_LARGEST = 1, 2, 4
 M3DRT_RATES_SCAT, M3DRT_RATES_FLAGS = 8, 16
-M3DRT_BBOP_LTE, M3DRT_BBOP_SPLIT = 1, 2
+M3DRT_BBOP_LTE, M3DRT_BBOP_SPLIT, M3DRT_BBOP_TRACK = 1, 2, 4
 
 BB_FIELDS = ("iblue", "ired", "lev_i", "lev_j", "Aij", "Bij", "lower_off", "q", "wnu", "wq", "g", "b",
              "nstar", "pop_ratio", "inv_df", "vproj", "e_kT", "adamp", "Inu", "Psi", "Bnu", "beta")
@@ -568,9 +568,10 @@ def _ali_lib():
     L = lib()
     if not getattr(L, "_ali_ok", False):
         L.m3drt_bb_rates.argtypes = [C.c_void_p, C.POINTER(BbRatesArgs)]
+        L.m3drt_bb_rates_window.argtypes = [C.c_void_p, C.POINTER(BbRatesArgs), C.c_void_p]
         L.m3drt_bb_opacity.argtypes = [C.c_void_p, C.POINTER(BbOpacityArgs)]
         L.m3drt_bf_rates.argtypes = [C.c_void_p, C.POINTER(BfRatesArgs)]
-        for n in ("m3drt_bb_rates", "m3drt_bb_opacity", "m3drt_bf_rates"):
+        for n in ("m3drt_bb_rates", "m3drt_bb_rates_window", "m3drt_bb_opacity", "m3drt_bf_rates"):
             getattr(L, n).restype = C.c_int
         L._ali_ok = True
     return L
@@ -601,6 +602,23 @@ def _bb_rates(self, d, wmu, wtot, gamma_ij, gamma_ji, precond=False, own_norm=Fa
     (ncell, nf) in the reference layout; gamma_ij, gamma_ji (nline, ncell) float32 are
     accumulated in place.  With largest and precond, split holds SPLIT_FIELDS (psi
     flags when it holds ntrans, psi_flags_in and psi_flags_out, which is OR-ed into)."""
+    L, a = _bb_rates_args(d, wmu, wtot, gamma_ij, gamma_ji, precond, own_norm, largest, layout, split, split_offset)
+    self._bind_stream()
+    _check(L.m3drt_bb_rates(self._h, C.byref(a)), "m3drt_bb_rates")
+
+
+def _bb_rates_window(self, d, chi_cont, wmu, wtot, gamma_ij, gamma_ji, own_norm=False, layout="native", split=None,
+                     split_offset=0):
+    """bb_rates with largest and precond of a window that window_opacity formed from the
+    continuum opacity chi_cont: the tracked contributions are formed again from it, and
+    split holds only Irem, escape and chi (and the scattering and psi-flag arrays)."""
+    L, a = _bb_rates_args(d, wmu, wtot, gamma_ij, gamma_ji, True, own_norm, True, layout, split, split_offset)
+    _f32_like(d["Inu"], chi_cont)
+    self._bind_stream()
+    _check(L.m3drt_bb_rates_window(self._h, C.byref(a), _p(chi_cont)), "m3drt_bb_rates_window")
+
+
+def _bb_rates_args(d, wmu, wtot, gamma_ij, gamma_ji, precond, own_norm, largest, layout, split, split_offset):
     L = _ali_lib()
     sp = split or {}
     _check_dev(d, BB_DTYPES, "bb_rates")
@@ -617,8 +635,7 @@ def _bb_rates(self, d, wmu, wtot, gamma_ij, gamma_ji, precond=False, own_norm=Fa
     npw = int(sp["psi_flags_in"].shape[0]) if sp.get("psi_flags_in") is not None else 0
     a = BbRatesArgs(nline, nf, ncell, nk, flags, wmu, wtot, sf, sc, *[_p(d.get(k)) for k in BB_FIELDS],
                     _p(gamma_ij), _p(gamma_ji), split_offset, npw, *[_p(sp.get(k)) for k in SPLIT_FIELDS])
-    self._bind_stream()
-    _check(L.m3drt_bb_rates(self._h, C.byref(a)), "m3drt_bb_rates")
+    return L, a
 
 
 def _bb_opacity(self, d, xhat, ehat, wmu=0.0, lte=False, split=None, split_offset=0, wphi_line=None, wphi=None,
@@ -651,11 +668,12 @@ class WindowArgs(C.Structure):
 
 
 def _window_opacity(self, d, chi_cont, Bnu, beta, xhat, ehat, split=None, split_offset=0, lte=False,
-                    suppress_masers=False, maser_chi_floor=1e-4, n_floored=None, layout="native"):
+                    suppress_masers=False, maser_chi_floor=1e-4, n_floored=None, layout="native", track=False):
     """One direction's opacity pass over a window in one kernel (m3drt_window_opacity):
     the continuum, convert_to_work_units, the split tracking seeded with the continuum,
     the lines with add_largest, and work_to_transfer_units.  xhat receives chi and
-    ehat S; split (the six tracking arrays) is overwritten."""
+    ehat S; split (the six tracking arrays) is overwritten.  track: the same chi and S
+    without writing tracking arrays (bb_rates_window forms them again)."""
     L = _ali_lib()
     if not getattr(L, "_win_ok", False):
         L.m3drt_window_opacity.argtypes = [C.c_void_p, C.POINTER(BbOpacityArgs), C.POINTER(WindowArgs)]
@@ -668,7 +686,8 @@ def _window_opacity(self, d, chi_cont, Bnu, beta, xhat, ehat, split=None, split_
     nline, nf = d["q"].shape
     nk, ncell = d["nstar"].shape
     sf, sc = _strides(layout, nf, ncell)
-    flags = (M3DRT_BBOP_LTE if lte else 0) | (M3DRT_BBOP_SPLIT if split is not None else 0)
+    flags = ((M3DRT_BBOP_LTE if lte else 0) | (M3DRT_BBOP_SPLIT if split is not None else 0)
+             | (M3DRT_BBOP_TRACK if track else 0))
     a = BbOpacityArgs(nline, nf, ncell, nk, flags, split_offset, 0.0, sf, sc,
                       *[_p(d.get(k)) for k in ("iblue", "ired", "lev_i", "lev_j", "Bij", "lower_off", "q")], None,
                       None, *[_p(d.get(k)) for k in ("b", "nstar", "pop_ratio", "inv_df", "vproj", "e_kT", "adamp")],
@@ -699,6 +718,7 @@ def _bf_rates(self, d, nline, gamma_ij, gamma_ji, precond=False, cut_x=70.0, lay
 
 
 Context.bb_rates = _bb_rates
+Context.bb_rates_window = _bb_rates_window
 Context.bb_opacity = _bb_opacity
 Context.window_opacity = _window_opacity
 Context.bf_rates = _bf_rates

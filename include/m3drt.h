@@ -375,10 +375,18 @@ typedef struct {
  * skipped. */
 int m3drt_bb_rates(m3drt_ctx *ctx, const m3drt_bb_rates_args *args);
 
+/* m3drt_bb_rates with M3DRT_RATES_LARGEST | M3DRT_RATES_PRECOND of a window whose chi, S
+ * came from m3drt_window_opacity with the same lines, cells and chi_cont (f, cell), Bnu
+ * and beta: the tracked contributions are formed again from those, the same values
+ * that M3DRT_BBOP_SPLIT would have written, and the six split_ arrays are not used
+ * (NULL).  Line scattering and psi flags as there. */
+int m3drt_bb_rates_window(m3drt_ctx *ctx, const m3drt_bb_rates_args *args, const float *chi_cont);
+
 /* ------------------------------------------------------------------ line opacity of a model atom */
 
 #define M3DRT_BBOP_LTE 1    /* b = 1 (the LTE companion set) */
 #define M3DRT_BBOP_SPLIT 2  /* track the largest contribution per point (add_largest) */
+#define M3DRT_BBOP_TRACK 4  /* m3drt_window_opacity: as SPLIT, but the tracking arrays are not written */
 
 typedef struct {
   int32_t nline, nf, ncell, nk, flags, split_offset;

@@ -107,6 +107,68 @@ def test_window_opacity_equals_the_sequence(ctx, kw):
                 assert torch.equal(out[0][k], out[1][k]), (wi, r, k, float((out[0][k] - out[1][k]).abs().max()))
 
 
+def _overlapping(p, w, seed):
+    """The window's lines with windows that overlap: every line's start drawn anew, so
+    that a frequency holds none, one or several lines."""
+    g = np.random.default_rng(seed)
+    nline, nf, nq = len(w.lines), w.nf, p.cfg.nq
+    const = {k: v.clone() for k, v in w.const.items()}
+    q = np.linspace(-p.cfg.qmax, p.cfg.qmax, nq).astype(np.float32)
+    const["q"].zero_()
+    for l in range(nline):
+        f0 = int(g.integers(0, nf - nq + 1))
+        const["iblue"][l], const["ired"][l] = f0 + 1, f0 + nq
+        const["q"][l, f0:f0 + nq] = torch.from_numpy(q).cuda()
+        const["wnu"][l] = 1.0 / nq
+        const["wq"][l] = 2.0 * p.cfg.qmax / nq
+    return const
+
+
+@pytest.mark.parametrize("kw,overlap,off", [({}, False, 0), (dict(nq=50, lines_per_window=4), True, 3),
+                                            (dict(nq=7, nline=70, lines_per_window=70, nbound=20), True, 0)])
+def test_rates_with_the_tracking_formed_again(ctx, kw, overlap, off):
+    """window_opacity(track) and bb_rates_window against window_opacity with its tracking
+    arrays and bb_rates reading them: chi, S and the rate sums bit for bit, with lines
+    alone at their frequencies and overlapping, and with more lines than the covering
+    mask holds."""
+    from dispatch_amd.ali import NlteProblem
+    from dispatch_amd import synth
+    p = NlteProblem(ctx, small(**kw))
+    g = torch.Generator(device="cuda").manual_seed(5)
+    p.b.mul_(torch.exp(0.3 * torch.randn(p.b.shape, generator=g, dtype=torch.float64, device="cuda")))
+    print(f"rates with the tracking formed again {kw} overlap={overlap}", flush=True)
+    w = p.windows[0]
+    l0, l1, nf, nc = w.lines[0], w.lines[-1] + 1, w.nf, p.ncell
+    const = _overlapping(p, w, 4) if overlap else w.const
+    vproj = (p.vz * (p.vec[0][2] / synth.C_LIGHT)).float().contiguous()
+    d = dict(const, vproj=vproj, b=p.b, nstar=p.nstar, pop_ratio=p.pop_ratio, inv_df=p.inv_df, e_kT=p.e_kT32,
+             adamp=p.adamp[l0:l1])
+    rnd = lambda: torch.rand((nf, nc), generator=g, device="cuda")
+    Irem, esc, I = rnd() * w.Bnu, rnd(), rnd() * w.Bnu
+    out = []
+    for retrack in (False, True):
+        chi, S = torch.empty_like(w.chi_c), torch.empty_like(w.chi_c)
+        sp = {}
+        if not retrack:
+            sp = {k: torch.empty_like(w.chi_c) for k in ("split_opac1", "split_opac2", "split_chi1", "split_chi2")}
+            sp.update({k: torch.empty((nf, nc), dtype=torch.int32, device="cuda") for k in ("split_id", "split_chi_id")})
+        ctx.window_opacity(d, w.chi_c, w.Bnu, w.beta, chi, S, split=None if retrack else sp, split_offset=off,
+                           track=retrack)
+        Psi = torch.where(I < 0.05 * w.Bnu, torch.zeros_like(chi), esc / chi.abs())
+        gij, gji = torch.zeros((l1 - l0, nc), device="cuda"), torch.zeros((l1 - l0, nc), device="cuda")
+        dr, parts = dict(d, Inu=I, Psi=Psi, Bnu=w.Bnu, beta=w.beta), dict(sp, Irem=Irem, escape=esc, chi=chi)
+        if retrack:
+            ctx.bb_rates_window(dr, w.chi_c, 0.3, 1.0, gij, gji, own_norm=True, split=parts, split_offset=off)
+        else:
+            ctx.bb_rates(dr, 0.3, 1.0, gij, gji, precond=True, largest=True, own_norm=True, split=parts,
+                         split_offset=off)
+        out.append((chi, S, gij, gji))
+    torch.cuda.synchronize()
+    assert float(out[0][2].abs().max()) > 0
+    for a, b, what in zip(*out, ("chi", "S", "gamma_ij", "gamma_ji")):
+        assert torch.equal(a, b), (what, float((a - b).abs().max()))
+
+
 def test_graph_replays_of_the_rate_pass_match_eager(ctx):
     """AliConfig(graph=True): the rate pass captured once and replayed, with the
     statistical-equilibrium update (eager work) between the replays, gives the eager
