@@ -15,8 +15,9 @@
 //  * the cubes are read at a per-thread 32-bit offset that never changes from
 //    plane to plane against a wave-uniform base per (plane, row);
 //  * dt500 and 1/chi500 of a cell come as one pair.
-// The strips are exact (ny = L * strips, L from the instantiated set), so every
-// per-cell branch is resolved at compile time.
+// Every strip holds L rows (L from the instantiated set), so every per-cell branch is
+// resolved at compile time: ny = L * strips, or a last strip that starts at row ny - L
+// and leaves its first rows to the strip before it.
 #include "sweep_sc2.hpp"
 #include <cstdio>
 #include <cstdlib>
@@ -125,7 +126,11 @@ constexpr int fast_max_threads() { return L >= 30 ? 512 : L >= 20 ? 768 : 1024; 
 // form writes them for a cell without eta flags (SRC/rt_solvers_mod.f90:419-440,
 // 465-475; the maser limit on |I| before the clamp); 2, no J: every cell's I (the
 // intensity cube an adjoint sweep recomputes).
-template <int L, bool PJ, int MODE, int CPL, int SR = 0, int OM = 0>
+// RAG: any ny >= L.  The last strip starts at row ny - L, so that every strip holds L
+// rows and the cell loop stays straight-line; its first `skip` rows belong to the strip
+// before it, and their stores fall away (global ones beyond the buffer's size, LDS ones
+// masked).
+template <int L, bool PJ, int MODE, int CPL, int SR = 0, int OM = 0, bool RAG = false>
 __global__ void __launch_bounds__(fast_max_threads<L>()) sc2_fast(const FastArgs<float> a) {
   using namespace dev;
   using T = float;
@@ -134,10 +139,11 @@ __global__ void __launch_bounds__(fast_max_threads<L>()) sc2_fast(const FastArgs
   // rows of loads in flight ahead of the row being computed (two cells' loads per
   // step with CPL = 2).  4 measured best for strips of 15 and 20 rows on the
   // 120 x 120 plane (13.3 ms against 13.9 with 3 and 14.1 with 6 for strips of 20).
-  constexpr int PD = CPL == 1 ? (L >= 15 ? 4 : 3) : 1;
+  constexpr int PD = CPL == 1 ? (L >= 15 && !(RAG && PJ) ? 4 : L < 3 ? L : 3) : 1;
   constexpr uint32_t TB = sizeof(T);
   static_assert(MODE != 4 || (CPL == 1 && SR >= 1 && SR <= L), "S rows in LDS: one column per lane, SR <= L");
   constexpr bool SPL = OM == 1, IOUT = OM >= 1;
+  static_assert(!RAG || (CPL == 1 && MODE != 4 && L >= 2), "short last strips: one column per lane, no S rows");
   static_assert(OM == 0 || (CPL == 1 && !PJ && MODE != 4), "cell outputs: one column per lane, no PsiJ, S rows whole");
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int nx = a.nx, ny = a.ny, PW = a.PW, nxy = nx * ny;
@@ -150,7 +156,8 @@ __global__ void __launch_bounds__(fast_max_threads<L>()) sc2_fast(const FastArgs
   const int nxp = nx / CPL;
   const int x0 = (tid % nxp) * CPL;
   const int strip = tid / nxp;
-  const int yb = strip * L;
+  const int yb = RAG ? min(strip * L, ny - L) : strip * L;
+  const int skip = RAG ? strip * L - yb : 0;
   const int rb = (yb + a.yo + 2) * PW + (x0 + a.xo + 2);  // row 0 of the window, padded index
   int xc[CPL + 1];                                        // upwind columns of S (wrapped)
 #pragma unroll
@@ -190,6 +197,9 @@ __global__ void __launch_bounds__(fast_max_threads<L>()) sc2_fast(const FastArgs
     }
     return P;
   };
+  // row k's store offset; beyond the buffer for a row of another strip (the range check
+  // of a raw buffer drops the store)
+  auto sto = [&](int k) -> uint32_t { return RAG && k < skip ? 0x80000000u : voff; };
   const uint32_t rowb = a.cs_y * TB, drowb = nx * (uint32_t)sizeof(Pair<T>);
   auto fetch = [&](const Planes &P, int k) -> In {
     In v;
@@ -348,14 +358,14 @@ __global__ void __launch_bounds__(fast_max_threads<L>()) sc2_fast(const FastArgs
           PJn.v[c] = in.PsJ.v[c] + a.wj * psiout;
         }
       }
-      if (IOUT) bst<V>(P.Io, voff, k * rowb, Io);
+      if (IOUT) bst<V>(P.Io, sto(k), k * rowb, Io);
       if (SPL) {
-        bst<V>(P.Po, voff, k * rowb, Po);
-        bst<V>(P.Ro, voff, k * rowb, Ro);
-        bst<V>(P.Eo, voff, k * rowb, Eo);
+        bst<V>(P.Po, sto(k), k * rowb, Po);
+        bst<V>(P.Ro, sto(k), k * rowb, Ro);
+        bst<V>(P.Eo, sto(k), k * rowb, Eo);
       }
-      if (!IOUT) bst<V>(P.J, voff, k * rowb, Jn);
-      if (PJ) bst<V>(P.PsJ, voff, k * rowb, PJn);
+      if (!IOUT) bst<V>(P.J, sto(k), k * rowb, Jn);
+      if (PJ) bst<V>(P.PsJ, sto(k), k * rowb, PJn);
       w0 = w1;
       w1 = w2;
       w2 = w3;
@@ -391,10 +401,12 @@ __global__ void __launch_bounds__(fast_max_threads<L>()) sc2_fast(const FastArgs
       }
     };
 #pragma unroll
-    for (int k = 0; k < L; ++k) put(wb + k * PW, k);
+    for (int k = 0; k < L; ++k)
+      if (!RAG || k >= skip) put(wb + k * PW, k);
     if (xedge) {
 #pragma unroll
-      for (int k = 0; k < L; ++k) put(wb + k * PW + dh, k);
+      for (int k = 0; k < L; ++k)
+        if (!RAG || k >= skip) put(wb + k * PW + dh, k);
     }
     if (strip == 0) {
 #pragma unroll
@@ -406,9 +418,15 @@ __global__ void __launch_bounds__(fast_max_threads<L>()) sc2_fast(const FastArgs
     if (strip == a.nstrips - 1) {
 #pragma unroll
       for (int k = L - 2; k < L; ++k) {
+        if (RAG && k < skip) continue;
         put(wb + (k - ny) * PW, k);
         if (xedge) put(wb + (k - ny) * PW + dh, k);
       }
+    }
+    // a last strip of one row: row ny - 2 is the last of the strip before it
+    if (RAG && strip == a.nstrips - 2 && yb + L == ny - 1) {
+      put(wb + (L - 1 - ny) * PW, L - 1);
+      if (xedge) put(wb + (L - 1 - ny) * PW + dh, L - 1);
     }
     if (MODE == 4) {
       // row yb+k is window row k-yo of this strip (slot strip*SR + k-yo-1 while
@@ -432,7 +450,7 @@ __global__ void __launch_bounds__(fast_max_threads<L>()) sc2_fast(const FastArgs
 #pragma unroll
       for (int k = 0; k < L; ++k) {
         if (CPL == 1) {
-          bst<T>(ex, eo, k * a.gs_y * TB, newI[0][k]);
+          bst<T>(ex, RAG && k < skip ? 0x80000000u : eo, k * a.gs_y * TB, newI[0][k]);
         } else {
           V ev;
 #pragma unroll
@@ -445,9 +463,9 @@ __global__ void __launch_bounds__(fast_max_threads<L>()) sc2_fast(const FastArgs
   }
 }
 
-template <int L, bool PJ, int MODE, int CPL, int SR = 0, int OM = 0>
+template <int L, bool PJ, int MODE, int CPL, int SR = 0, int OM = 0, bool RAG = false>
 int launch_fast(m3drt_ctx *ctx, const FastArgs<float> &a, int nf, int nt, size_t lds) {
-  auto kern = sc2_fast<L, PJ, MODE, CPL, SR, OM>;
+  auto kern = sc2_fast<L, PJ, MODE, CPL, SR, OM, RAG>;
   M3DRT_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   hipLaunchKernelGGL(kern, dim3(nf), dim3(nt), lds, ctx->stream, a);
   M3DRT_HIP(hipGetLastError());
@@ -487,6 +505,37 @@ int fast_variant(m3drt_ctx *ctx, const FastArgs<float> &a, int nf, int nt, int m
     if (mode == 4 && sr == 8) return launch_fast<L, false, 4, CPL, 8>(ctx, a, nf, nt, l4);
   }
   return launch_fast<L, false, 1, CPL>(ctx, a, nf, nt, l2);
+}
+
+// the forms with a short last strip: every output, one column per lane, modes 1 and 2
+template <int L>
+int rag_variant(m3drt_ctx *ctx, const FastArgs<float> &a, int nf, int nt, int mode, size_t np) {
+  const size_t l2 = np * 2 * sizeof(float), l3 = np * 3 * sizeof(float);
+  if (a.Psiout) {
+    if (mode == 2) return launch_fast<L, false, 2, 1, 0, 1, true>(ctx, a, nf, nt, l3);
+    return launch_fast<L, false, 1, 1, 0, 1, true>(ctx, a, nf, nt, l2);
+  }
+  if (a.Iout) {
+    if (mode == 2) return launch_fast<L, false, 2, 1, 0, 2, true>(ctx, a, nf, nt, l3);
+    return launch_fast<L, false, 1, 1, 0, 2, true>(ctx, a, nf, nt, l2);
+  }
+  if (a.PsiJ) {
+    if (mode == 2) return launch_fast<L, true, 2, 1, 0, 0, true>(ctx, a, nf, nt, l3);
+    return launch_fast<L, true, 1, 1, 0, 0, true>(ctx, a, nf, nt, l2);
+  }
+  if (mode == 2) return launch_fast<L, false, 2, 1, 0, 0, true>(ctx, a, nf, nt, l3);
+  return launch_fast<L, false, 1, 1, 0, 0, true>(ctx, a, nf, nt, l2);
+}
+
+constexpr int kRag[] = {2, 4, 8, 12, 20};
+
+int rag_dispatch(m3drt_ctx *ctx, const FastArgs<float> &a, int nf, int nt, int L, int mode, size_t np) {
+  if (L == 2) return rag_variant<2>(ctx, a, nf, nt, mode, np);
+  if (L == 4) return rag_variant<4>(ctx, a, nf, nt, mode, np);
+  if (L == 8) return rag_variant<8>(ctx, a, nf, nt, mode, np);
+  if (L == 12) return rag_variant<12>(ctx, a, nf, nt, mode, np);
+  if (L == 20) return rag_variant<20>(ctx, a, nf, nt, mode, np);
+  return -1;
 }
 
 // strip lengths instantiated: one lane per column (60, 96, 120-cell planes), two
@@ -549,7 +598,7 @@ int run_fast(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const m3drt_sweep_bufs *
   const int want = lenv ? atoi(lenv) : 0;
   auto max_threads = [](int l) { return l >= 30 ? 512 : l >= 20 ? 768 : 1024; };
   int L = 0;
-  if (!want && cpl == 1 && ny % 20 == 0 && ny / 20 >= 2 && (ny / 20) * nx >= 512 && (ny / 20) * nx <= 768) L = 20;
+  if (!want && !L && cpl == 1 && ny % 20 == 0 && ny / 20 >= 2 && (ny / 20) * nx >= 512 && (ny / 20) * nx <= 768) L = 20;
   // Where the pairs and S of three workgroups fit one CU's LDS, a strip of 15 (or 20)
   // rows that still gives a workgroup more than three waves: four rows of loads in
   // flight instead of three, three workgroups per CU.  On the 60 x 60 plane the
@@ -570,24 +619,64 @@ int run_fast(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const m3drt_sweep_bufs *
     }
     if (!L && cpl == 2) cpl = 1;
   }
-  if (!L) return -1;
-  const int nstrips = ny / L;
-  const int nt = (nx / cpl) * nstrips;
-  const size_t np = (size_t)(nx + 4) * (ny + 4);
   const uint64_t span = (uint64_t)(nx - 1) * d->cs_x + (uint64_t)(ny - 1) * d->cs_y;
   const uint64_t gspan = (uint64_t)(nx - 1) * d->gs_x + (uint64_t)(ny - 1) * d->gs_y;
   if ((span + 1) * sizeof(T) >= (1ull << 32) || (gspan + 1) * sizeof(T) >= (1ull << 32)) return -1;
+  // Strips that need not divide ny.  The one taken leaves the fewest rounds of
+  // workgroups, and among those the shortest strips: a workgroup's plane takes about
+  // 0.75 + 0.27 L us where the memory is not the limit.  cap: the threads a CU holds at
+  // the kernel's register use.  Measured (J, 30 planes, L = 2 / 4 / 8 / 12 us, then the
+  // general kernel): 40 x 41 x 250 frequencies 67 / 70 / 87 / 117, 112; 40 x 41 x 800
+  // 253 / 192 / 195 / 214, 451; 60 x 59 x 480 - / 236 / 216 / 222, 380; 101 x 67 x 250
+  // (46 planes) - / - / 353 / 356, 495.
+  const char *renv = getenv("M3DRT_FAST_RAG");
+  const int rwant = renv ? atoi(renv) : 0;
+  int Lr = 0;
+  if (cpl == 1 && !want && !getenv("M3DRT_NO_RAG") && (span + 1) * sizeof(T) < (1ull << 31) && (gspan + 1) * sizeof(T) < (1ull << 31)) {
+    const size_t lds = np_all * (3 * np_all * sizeof(T) <= (size_t)ctx->lds_max ? 3 : 2) * sizeof(T);
+    int best = 0;
+    for (int c : kRag) {
+      const int t = (ny + c - 1) / c * nx, cap = c <= 2 ? 2048 : c <= 4 ? 1536 : c <= 12 ? 1024 : 768;
+      // (with PsiJ strips of 20 spill: 556 us against the general kernel's 500 on
+      // 118 x 110 x 250, 1085 against 1002 on 117 x 113 x 500, 23 planes)
+      if (c == 20 && get_rates && b->PsiJ && !rwant) continue;
+      if (c + 2 > ny || t > max_threads(c) || lds > (size_t)ctx->lds_max || (rwant && c != rwant)) continue;
+      const int wgs = std::max(1, std::min(cap / t, (int)((size_t)ctx->lds_max / lds)));
+      const int rounds = (d->nf + 256 * wgs - 1) / (256 * wgs);
+      if (!Lr || rounds < best) {
+        Lr = c;
+        best = rounds;
+      }
+    }
+  }
+  // Where a longer strip divides ny: that form, but on few points, where the shorter
+  // strips' latency counts (30 planes, us): 60 x 60 x 60 frequencies 96 with strips of 4
+  // against 123 with 15, 60 x 60 x 250 120 against 132, 12 x 30 x 64 (20 planes) 27 with 2
+  // against 102 with 15; 60 x 60 x 480 216 with 8 against 207 with 15, 110 x 75 x 250 (23
+  // planes) 232 with 12 against 212 with 15.  Strips of 2 for 4: 33 x 12 x 64 38 against
+  // 50, 13 x 100 x 200 67 against 74, but with PsiJ 14 x 104 x 421 5 % slower.
+  // (From 8 frequencies on; fewer were not measured and keep the strip that divides.)
+  // Strips of 4 that tile ny but fit a CU at most twice and leave another round of
+  // workgroups: the longer ones (48 x 48 x 1000 265 with 12 against 312).
+  const int64_t pts = (int64_t)nx * ny * d->nf;
+  const bool rag = Lr && (!L || rwant || (Lr < L && d->nf >= 8 && pts < (L == 4 ? 180000 : 1300000)) ||
+                          (L == 4 && Lr > 4 && ny / 4 * nx > 512));
+  if (rag) L = Lr;
+  if (!L) return -1;
+  const int nstrips = (ny + L - 1) / L;
+  const int nt = (nx / cpl) * nstrips;
+  const size_t np = (size_t)(nx + 4) * (ny + 4);
   int mode = -1, sr = 0;
   if (np * 3 * sizeof(T) <= (size_t)ctx->lds_max) {
     mode = 2;
   } else if (np * 2 * sizeof(T) <= (size_t)ctx->lds_max) {
     mode = 1;
     // S of the first sr tap rows of every strip (nstrips * sr rows of nx, and a
-    // spare row) in the LDS the pairs leave: J only, one column per lane, strips of
+    // spare row) in the LDS the pairs leave: J only, one column per lane, exact strips of
     // 20 rows (the form that holds it without spilling registers)
     const size_t rows = ((size_t)ctx->lds_max - np * 2 * sizeof(T)) / ((size_t)nx * sizeof(T));
     const bool j_only = !(get_rates && b->PsiJ) && !spl && !iout;
-    if (j_only && cpl == 1 && L == 20 && rows >= 1 && !getenv("M3DRT_FAST_NO_SROWS")) {
+    if (j_only && cpl == 1 && L == 20 && !rag && rows >= 1 && !getenv("M3DRT_FAST_NO_SROWS")) {
       // the most rows per strip to hold: 8 unless M3DRT_FAST_SR says otherwise.  On
       // the 120 x 120 plane, per 1024-frequency direction: 13.35 ms with 8 and 13.45
       // with 14 over all 24 directions, 13.32 and 13.10 over four of them on another
@@ -647,10 +736,11 @@ int run_fast(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const m3drt_sweep_bufs *
   a.wj = (T)d->wj;
   if (getenv("M3DRT_VERBOSE"))
     fprintf(stderr, "[m3drt] sc2 fast %s nf=%d plane=%dx%d nz=%d: %d threads, %d column(s) per lane, strip %d, "
-            "LDS mode %d (%zu B, %d S rows of %d per strip in LDS)%s\n", f64 ? "f64" : "f32", d->nf, nx, ny, nz,
+            "LDS mode %d (%zu B, %d S rows of %d per strip in LDS)%s%s\n", f64 ? "f64" : "f32", d->nf, nx, ny, nz,
             nt, cpl, L, mode,
             np * (mode == 2 ? 3 : 2) * sizeof(T) + (mode == 4 ? (size_t)(nstrips * sr + 1) * nx * sizeof(T) : 0),
-            mode == 2 ? L + 1 : sr, L + 1, a.PsiJ ? ", PsiJ" : spl ? ", split outputs" : iout ? ", I out" : "");
+            mode == 2 ? L + 1 : sr, L + 1, rag ? ", short last strip" : "", a.PsiJ ? ", PsiJ" : spl ? ", split outputs" : iout ? ", I out" : "");
+  if (rag) return rag_dispatch(ctx, a, d->nf, nt, L, mode, np);
   return fast_dispatch(ctx, a, d->nf, nt, L, cpl, mode, np, sr);
 }
 

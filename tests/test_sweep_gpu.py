@@ -440,3 +440,39 @@ def test_sweep_plane_form_matches_oracle(ctx, monkeypatch, rows, nf, nx, ny, nz,
                  d(case["I"][gz]), d(case["chi500"]), d(case["chi500_up"]), d(case["g500"]), dir=case["dir"],
                  ds=case["ds"], vec=case["vec"], layout="reference", wj=0.25, J=Jd)
     check32(Jd.cpu().numpy(), 0.125 + 0.25 * interior(run_oracle(case)[0]).astype(np.float64), "J alone")
+
+
+# the straight-line sweep with a last strip that leaves its first rows to the strip
+# before it: none, one and all but one of its rows left, two and more strips, planes as
+# narrow as the kernel takes, S in LDS and (the widest) from the cache
+@pytest.mark.parametrize("rows,nx,ny,nz,vec", [
+    (2, 4, 4, 3, (0.3, -0.4, 0.866)), (2, 9, 5, 4, (-0.5, 0.2, -0.84)), (4, 5, 7, 4, (0.1, 0.97, 0.211)),
+    (4, 12, 9, 3, (-0.4, 0.5, 0.7)), (8, 7, 13, 3, (0.61481017, 0.0, 0.78867513)), (8, 6, 17, 3, (0.4, -0.5, -0.7)),
+    (12, 5, 25, 3, (0.9, 0.2, 0.39)), (12, 17, 23, 2, (-0.9, -0.2, -0.39)), (20, 6, 41, 2, (0.3, -0.4, 0.866)),
+    (20, 4, 22, 2, (-0.3, 0.4, -0.866)), (20, 117, 113, 2, (0.3, 0.4, 0.866)),
+])
+def test_sweep_short_last_strip_matches_oracle(ctx, monkeypatch, rows, nx, ny, nz, vec):
+    monkeypatch.setenv("M3DRT_FAST_RAG", str(rows))
+    nf = 3
+    case = make_case(nf=nf, nx=nx, ny=ny, nz=nz, seed=rows + ny, vec=vec, maser=ny == 25)
+    print(f"short last strip rows={rows} plane={nx}x{ny} nz={nz}", flush=True)
+    I, psi, irem, esc = run_oracle(case, split_rates=True)
+    psi1 = run_oracle(case)[1]
+    Iref = interior(I).astype(np.float64)
+    last = case["nz"] if case["dir"] > 0 else 1
+    gz = case["gz"]
+    c, s = dev(to_native(interior(case["chi"]))), dev(to_native(interior(case["S"])))
+    gh = [dev(plane_to_native(case[k][gz])) for k in ("chi", "S", "I")]
+    new = lambda v: torch.full_like(c, v)
+    back = lambda t: np.moveaxis(t.double().cpu().numpy(), 1, 3)
+    for outs in (("J",), ("J", "PsiJ"), ("I_out",), ("I_out", "Psi_out", "Irem_out", "escape_out"), ()):
+        o = {k: new(0.125 if k in ("J", "PsiJ") else 0.0) for k in outs}
+        ex = torch.zeros_like(gh[0])
+        ctx.sc_sweep(c, s, *gh, dev(case["chi500"]), dev(case["chi500_up"]), dev(case["g500"]), dir=case["dir"],
+                     ds=case["ds"], vec=case["vec"], wj=0.25, exit_I=ex, split_rates="Irem_out" in outs,
+                     get_rates="PsiJ" in outs or "Psi_out" in outs, **o)
+        ref = dict(J=0.125 + 0.25 * Iref, PsiJ=0.125 + 0.25 * psi1.astype(np.float64), I_out=Iref, Psi_out=psi,
+                   Irem_out=irem, escape_out=esc)
+        for k, t in o.items():
+            check32(back(t), ref[k], f"{k} of {outs}")
+        check32(np.moveaxis(ex.double().cpu().numpy(), 0, 2), I[last], f"exit plane of {outs}")
