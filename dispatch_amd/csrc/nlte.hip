@@ -5,13 +5,18 @@
 // under-relaxation, particle conservation, population floor and the convergence
 // measure.  Also the rate normalisation of normalize_profiles (377-431).
 //
-// Mapping.  One thread per cell.  A workgroup of NT cells keeps every cell's
-// nk x nk matrix, right-hand side and b*n* vector in LDS, interleaved cell-fastest
-// (element e of cell t at e*NT + t), so the lanes of a wavefront touch
-// consecutive doubles and the in-place elimination runs without bank conflicts.
+// Mapping.  Sixteen lanes per cell, four cells a wavefront.  A workgroup of NT cells
+// keeps every cell's nk x nk matrix, right-hand side and b*n* vector in LDS, one cell
+// after another.  A cell's lanes share its elimination as a 4 x 4 grid over the rows and
+// columns left, and otherwise take its levels in turn; they lie in one wavefront, whose
+// LDS accesses are in order, so no barrier is needed between the steps.  Every element
+// sees the operations of the sequential algorithm in its order, so the results are
+// those of one lane per cell.  What bounds it is the latency of the dependent steps
+// (LDS, FP64): a cell's matrix (3.9 KB at 21 levels) allows 40 cells a CU, which with one
+// lane each were a single wave.  432 000 cells of 21 levels: 12.7 -> 3.7 ms.
 // The atom (levels, transitions, pairs) is uniform and read through the scalar
 // cache.  The largest change and the per-level changes are reduced first per
-// workgroup and then by one workgroup, both keeping the first cell in the
+// workgroup and then by one workgroup each, both keeping the first cell in the
 // reference's loop order on ties, so the result is deterministic.
 #include "m3drt_internal.hpp"
 #include <cmath>
@@ -47,19 +52,31 @@ __device__ __forceinline__ bool better(double va, int ca, double vb, int cb) {
   return a > b || (a == b && ca < cb);
 }
 
-__global__ void __launch_bounds__(64) se_update_kernel(const SeArgs a) {
+constexpr int kSeLanes = 16;       // lanes of a cell
+constexpr int kSeCells = 40;       // cells of a workgroup, at most
+
+// doubles of a cell in LDS: matrix, right-hand side, b*n*; odd, so that the cells of a
+// wavefront start on different banks
+__host__ __device__ __forceinline__ int se_stride(int nk) { return (nk * nk + 2 * nk) | 1; }
+
+__global__ void __launch_bounds__(kSeLanes * kSeCells) se_update_kernel(const SeArgs a) {
   extern __shared__ double sm[];
   const int nk = a.nk, NT = a.nt;
-  const int t = threadIdx.x;
+  const int t = threadIdx.x / kSeLanes, p = threadIdx.x % kSeLanes;
   const int c = blockIdx.x * NT + t;
-  double *W = sm;                        // nk*nk*NT
-  double *E = W + (size_t)nk * nk * NT;  // nk*NT
-  double *BN = E + (size_t)nk * NT;      // nk*NT (b*n*, then b_old)
-  double *RV = BN + (size_t)nk * NT;     // 2*NT reduction values
-  int *RC = reinterpret_cast<int *>(RV + 2 * NT);  // 2*NT reduction cells
-#define Wm(i, j) W[((size_t)(i) * nk + (j)) * NT + t]
-#define Ev(i) E[(size_t)(i) * NT + t]
-#define Bv(i) BN[(size_t)(i) * NT + t]
+  double *W = sm + (size_t)t * se_stride(nk);    // nk*nk
+  double *E = W + (size_t)nk * nk;               // nk
+  double *BN = E + nk;                           // nk (b*n*, then b_old)
+  double *RV = sm + (size_t)NT * se_stride(nk);  // NT reduction values
+  int *RC = reinterpret_cast<int *>(RV + NT);    // NT cells, NT levels
+#define Wm(i, j) W[(i) * nk + (j)]
+#define Ev(i) E[i]
+#define Bv(i) BN[i]
+  // orders a cell's LDS accesses between its lanes (one wavefront: no barrier needed)
+  auto sync = [] {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
   const bool live = c < a.ncell && a.totn[c] > 0 && a.temp[c] < a.tmax_update;
   double my_err = 0.0;
   int my_lvl = -1;
@@ -67,87 +84,116 @@ __global__ void __launch_bounds__(64) se_update_kernel(const SeArgs a) {
   if (live) {
     const double ekt = a.e_kT[c];
     auto NS = [&](int i) { return a.nstar[(size_t)i * a.ncell + c]; };
-    for (int i = 0; i < nk; ++i) {
-      Ev(i) = 0.0;
-      for (int j = 0; j < nk; ++j) Wm(i, j) = 0.0;
-    }
-    for (int kr = 0; kr < a.nrad; ++kr) {
-      if (!a.active[kr]) continue;
-      const int i = a.ti[kr] - 1, j = a.tj[kr] - 1;
-      if ((a.ev[j] - a.ev[i]) * ekt > a.cut_x) {
-        // a detailed-balance pair for a transition beyond cut_x kT
-        const double cut = kr < a.nline ? a.Aji[kr] : a.bf_cut_rate;
-        Wm(i, j) = Wm(i, j) + cut;
-        Wm(j, i) = Wm(j, i) + cut * NS(j) / NS(i);
-        continue;
+    for (int e = p; e < nk * nk; e += kSeLanes) W[e] = 0.0;
+    for (int i = p; i < nk; i += kSeLanes) Ev(i) = 0.0;
+    sync();
+    // The rates of sixteen transitions at a time, one a lane, then added in their order:
+    // lane 0 the upward rate to W(j, i), lane 1 the downward one to W(i, j).
+    auto add = [&](int i, int j, double up, double down) {
+      if (i == j) {
+        if (p == 0) Wm(i, i) = (Wm(i, i) + up) + down;
+      } else if (p < 2) {
+        double *w = p ? &Wm(i, j) : &Wm(j, i);
+        *w = *w + (p ? down : up);
       }
-      double r_up, r_down;
-      if (kr < a.nline) {
-        const double th = a.gij[(size_t)kr * a.ncell + c], dev = a.gji[(size_t)kr * a.ncell + c];
-        const double g_ij = a.g[i] / a.g[j];
-        if (NS(i) > 0 && NS(j) > 0) {
-          const double beta = NS(j) * g_ij / NS(i);
-          r_up = th * (beta / (1.0 - beta)) + dev;
-          r_down = g_ij * (th / (1.0 - beta) + dev);
+      sync();
+    };
+    for (int k0 = 0; k0 < a.nrad; k0 += kSeLanes) {
+      const int kr = k0 + p;
+      double r_up = 0.0, r_down = 0.0;
+      if (kr < a.nrad && a.active[kr]) {
+        const int i = a.ti[kr] - 1, j = a.tj[kr] - 1;
+        if ((a.ev[j] - a.ev[i]) * ekt > a.cut_x) {
+          // a detailed-balance pair for a transition beyond cut_x kT
+          const double cut = kr < a.nline ? a.Aji[kr] : a.bf_cut_rate;
+          r_down = cut;
+          r_up = cut * NS(j) / NS(i);
+        } else if (kr < a.nline) {
+          const double th = a.gij[(size_t)kr * a.ncell + c], dev = a.gji[(size_t)kr * a.ncell + c];
+          const double g_ij = a.g[i] / a.g[j];
+          if (NS(i) > 0 && NS(j) > 0) {
+            const double beta = NS(j) * g_ij / NS(i);
+            r_up = th * (beta / (1.0 - beta)) + dev;
+            r_down = g_ij * (th / (1.0 - beta) + dev);
+          }
         } else {
-          r_up = 0.0;
-          r_down = 0.0;
+          r_up = a.gij[(size_t)kr * a.ncell + c];
+          r_down = a.gji[(size_t)kr * a.ncell + c];
         }
-      } else {
-        r_up = a.gij[(size_t)kr * a.ncell + c];
-        r_down = a.gji[(size_t)kr * a.ncell + c];
       }
-      Wm(j, i) = Wm(j, i) + r_up;
-      Wm(i, j) = Wm(i, j) + r_down;
+      for (int q = 0; q < kSeLanes && k0 + q < a.nrad; ++q) {
+        if (!a.active[k0 + q]) continue;
+        add(a.ti[k0 + q] - 1, a.tj[k0 + q] - 1, __shfl(r_up, q, kSeLanes), __shfl(r_down, q, kSeLanes));
+      }
     }
     if (a.cswitch > 0 && a.cup) {
-      for (int q = 0; q < a.npair; ++q) {
-        const int i = a.pi[q] - 1, j = a.pj[q] - 1;
-        const double cu = a.cup[(size_t)q * a.ncell + c];
-        if (cu == 0) continue;
-        Wm(j, i) = Wm(j, i) + cu * a.cswitch;
-        Wm(i, j) = Wm(i, j) + cu * (NS(i) / NS(j)) * a.cswitch;
+      for (int q0 = 0; q0 < a.npair; q0 += kSeLanes) {
+        const int q = q0 + p;
+        double up = 0.0, down = 0.0;
+        if (q < a.npair) {
+          const int i = a.pi[q] - 1, j = a.pj[q] - 1;
+          const double cu = a.cup[(size_t)q * a.ncell + c];
+          if (cu != 0) {
+            up = cu * a.cswitch;
+            down = cu * (NS(i) / NS(j)) * a.cswitch;
+          }
+        }
+        for (int m = 0; m < kSeLanes && q0 + m < a.npair; ++m)
+          add(a.pi[q0 + m] - 1, a.pj[q0 + m] - 1, __shfl(up, m, kSeLanes), __shfl(down, m, kSeLanes));
       }
     }
-    for (int i = 0; i < nk; ++i) {
+    for (int i = p; i < nk; i += kSeLanes) {
       double s = 0.0;
       for (int k = 0; k < nk; ++k) s += Wm(k, i);
       Wm(i, i) = -s;
-    }
-    int pos = 0;
-    for (int i = 0; i < nk; ++i) {
       Bv(i) = a.b[(size_t)i * a.ncell + c] * NS(i);
-      if (Bv(i) > Bv(pos)) pos = i;
     }
-    Ev(pos) = a.totn[c];
+    sync();
+    int pos = 0;
     for (int i = 0; i < nk; ++i)
-      for (int j = 0; j < nk; ++j) Wm(i, j) = Wm(i, j) * Bv(j);
-    for (int j = 0; j < nk; ++j) Wm(pos, j) = Bv(j);
+      if (Bv(i) > Bv(pos)) pos = i;
+    if (p == 0) Ev(pos) = a.totn[c];
+    for (int j = p; j < nk; j += kSeLanes) {
+      const double bj = Bv(j);
+      for (int i = 0; i < nk; ++i) Wm(i, j) = i == pos ? bj : Wm(i, j) * bj;
+    }
+    sync();
 
     // lineq_no_pivot: Doolittle without pivoting, zero upper entries skipped
+    const int pi = p >> 2, pj = p & 3;
     for (int k = 0; k < nk - 1; ++k) {
       const double akk = Wm(k, k);
-      for (int i = k + 1; i < nk; ++i) Wm(i, k) = Wm(i, k) / akk;
-      for (int j = k + 1; j < nk; ++j) {
+      for (int i = k + 1 + p; i < nk; i += kSeLanes) Wm(i, k) = Wm(i, k) / akk;
+      sync();
+      for (int j = k + 1 + pj; j < nk; j += 4) {
         const double akj = Wm(k, j);
         if (akj != 0)
-          for (int i = k + 1; i < nk; ++i) Wm(i, j) = Wm(i, j) - Wm(i, k) * akj;
+          for (int i = k + 1 + pi; i < nk; i += 4) Wm(i, j) = Wm(i, j) - Wm(i, k) * akj;
       }
+      sync();
     }
-    for (int i = 0; i < nk; ++i)
-      for (int j = 0; j < i; ++j) Ev(i) = Ev(i) - Wm(i, j) * Ev(j);
+    // forward by columns (each Ev(i) takes its terms in the order of j), backward by rows
+    // on every lane alike
+    for (int j = 0; j < nk - 1; ++j) {
+      const double ej = Ev(j);
+      for (int i = j + 1 + p; i < nk; i += kSeLanes) Ev(i) = Ev(i) - Wm(i, j) * ej;
+      sync();
+    }
     for (int i = nk - 1; i >= 0; --i) {
-      for (int j = i + 1; j < nk; ++j) Ev(i) = Ev(i) - Wm(i, j) * Ev(j);
-      Ev(i) = Ev(i) / Wm(i, i);
+      double e = Ev(i);
+      for (int j = i + 1; j < nk; ++j) e = e - Wm(i, j) * Ev(j);
+      e = e / Wm(i, i);
+      sync();
+      if (p == 0) Ev(i) = e;
+      sync();
     }
     bool finite = true;
     for (int i = 0; i < nk; ++i) finite = finite && (fabs(Ev(i)) <= 1.79769313486231570e308);
     if (!finite) {
-      atomicMin(a.status, c + 1);
+      if (p == 0) atomicMin(a.status, c + 1);
     } else {
       const double eup = a.max_update > 1.0 ? a.max_update : 1.0, elo = 1.0 / eup;
-      double sum = 0.0;
-      for (int i = 0; i < nk; ++i) {
+      for (int i = p; i < nk; i += kSeLanes) {
         double e = Ev(i);
         if (e < elo || e > eup) clamps++;
         if (e < elo)
@@ -155,70 +201,67 @@ __global__ void __launch_bounds__(64) se_update_kernel(const SeArgs a) {
         else if (e > eup)
           e = eup * (2.0 - eup / e);
         if (a.sor_w != 1.0) e = pow(e, a.sor_w);
-        const size_t o = (size_t)i * a.ncell + c;
-        const double bo = a.b[o];
+        const double bo = a.b[(size_t)i * a.ncell + c];
         Bv(i) = bo;                       // b_old
-        const double bn = bo * e;
-        Ev(i) = bn;                       // b, before normalisation
-        sum += bn * a.nstar[o];
+        Ev(i) = bo * e;                   // b, before normalisation
       }
+      sync();
+      double sum = 0.0;
+      for (int i = 0; i < nk; ++i) sum += Ev(i) * NS(i);
       const double norm = a.totn[c] / sum;
-      double wmax = -1.0;
-      for (int i = 0; i < nk; ++i) {
+      sync();
+      for (int i = p; i < nk; i += kSeLanes) {
         const size_t o = (size_t)i * a.ncell + c;
         double bn = Ev(i) * norm;
         if (a.nstar[o] > 0) bn = fmax(bn, fmin(1.0, a.min_pop_frac * a.totn[c] / a.nstar[o]));
         a.b[o] = bn;
         const double e = Bv(i) > 0 ? bn / Bv(i) - 1.0 : 0.0;
-        Ev(i) = e;                        // the change, for the per-level reduction
         double ew = fabs(e);
         if (a.conv_pop_floor > 0) ew = fabs(e) * fmin(1.0, bn * a.nstar[o] / (a.conv_pop_floor * a.totn[c]));
-        if (ew > wmax) {
-          wmax = ew;
+        Ev(i) = e;                        // the change, for the per-level reduction
+        Bv(i) = ew;
+      }
+      sync();
+      double wmax = -1.0;
+      for (int i = 0; i < nk; ++i)
+        if (Bv(i) > wmax) {
+          wmax = Bv(i);
           my_lvl = i;
         }
-      }
-      my_err = copysign(wmax, Ev(my_lvl));
+      // (my_lvl stays -1 where every change is NaN)
+      if (my_lvl >= 0) my_err = copysign(wmax, Ev(my_lvl));
     }
   }
   if (clamps) atomicAdd(a.nclamp, clamps);
 
-  // workgroup reduction: the largest weighted change, then every level's change
-  const int cell = (live && my_lvl >= 0) ? c : -1;
+  // workgroup reduction: the largest weighted change, and every level's change, one
+  // thread each
+  if (p == 0) {
+    RV[t] = my_err;
+    RC[t] = (live && my_lvl >= 0) ? c : -1;
+    RC[NT + t] = my_lvl;
+  }
+  __syncthreads();
   const int nblk = blockIdx.x;
-  __syncthreads();
-  RV[t] = my_err;
-  RC[t] = cell;
-  RC[NT + t] = my_lvl;
-  __syncthreads();
-  if (t == 0) {
+  for (int q = threadIdx.x; q <= nk; q += blockDim.x) {
     double bv = 0.0;
     int bc = -1, bl = -1;
-    for (int s = 0; s < NT; ++s)
-      if (better(RV[s], RC[s], bv, bc)) {
-        bv = RV[s];
-        bc = RC[s];
+    for (int s = 0; s < NT; ++s) {
+      const int cs = RC[s];
+      const double v = q == nk ? RV[s] : cs >= 0 ? sm[(size_t)s * se_stride(nk) + nk * nk + q] : 0.0;
+      if (better(v, cs, bv, bc)) {
+        bv = v;
+        bc = cs;
         bl = RC[NT + s];
       }
-    a.blk_err[nblk] = bv;
-    a.blk_cell[nblk] = bc;
-    a.blk_lvl[nblk] = bl;
-  }
-  for (int i = 0; i < nk; ++i) {
-    __syncthreads();
-    RV[t] = cell >= 0 ? Ev(i) : 0.0;
-    RC[t] = cell;
-    __syncthreads();
-    if (t == 0) {
-      double bv = 0.0;
-      int bc = -1;
-      for (int s = 0; s < NT; ++s)
-        if (better(RV[s], RC[s], bv, bc)) {
-          bv = RV[s];
-          bc = RC[s];
-        }
-      a.blk_lerr[(size_t)nblk * nk + i] = bv;
-      a.blk_lcell[(size_t)nblk * nk + i] = bc;
+    }
+    if (q == nk) {
+      a.blk_err[nblk] = bv;
+      a.blk_cell[nblk] = bc;
+      a.blk_lvl[nblk] = bl;
+    } else {
+      a.blk_lerr[(size_t)nblk * nk + q] = bv;
+      a.blk_lcell[(size_t)nblk * nk + q] = bc;
     }
   }
 #undef Wm
@@ -226,47 +269,44 @@ __global__ void __launch_bounds__(64) se_update_kernel(const SeArgs a) {
 #undef Bv
 }
 
-// the blocks' winners, reduced by one workgroup; out[0] = maxerr, out[1..nk] = lvlerr,
-// iout[0] = cell, iout[1] = level
+// the blocks' winners, one workgroup per value: workgroup 0 maxerr (out[0], its cell
+// iout[0] and level iout[1]), workgroup 1 + q level q (out[1 + q])
 __global__ void __launch_bounds__(256) se_final_kernel(int nblk, int nk, const double *blk_err,
                                                        const int32_t *blk_cell, const int32_t *blk_lvl,
                                                        const double *blk_lerr, const int32_t *blk_lcell,
                                                        double *out, int32_t *iout) {
   __shared__ double rv[256];
   __shared__ int rc[256], rl[256];
-  const int t = threadIdx.x;
-  for (int q = -1; q < nk; ++q) {
-    double bv = 0.0;
-    int bc = -1, bl = -1;
-    for (int s = t; s < nblk; s += blockDim.x) {
-      const double v = q < 0 ? blk_err[s] : blk_lerr[(size_t)s * nk + q];
-      const int cc = q < 0 ? blk_cell[s] : blk_lcell[(size_t)s * nk + q];
-      if (better(v, cc, bv, bc)) {
-        bv = v;
-        bc = cc;
-        bl = q < 0 ? blk_lvl[s] : q;
-      }
+  const int t = threadIdx.x, q = (int)blockIdx.x - 1;
+  double bv = 0.0;
+  int bc = -1, bl = -1;
+  for (int s = t; s < nblk; s += blockDim.x) {
+    const double v = q < 0 ? blk_err[s] : blk_lerr[(size_t)s * nk + q];
+    const int cc = q < 0 ? blk_cell[s] : blk_lcell[(size_t)s * nk + q];
+    if (better(v, cc, bv, bc)) {
+      bv = v;
+      bc = cc;
+      bl = q < 0 ? blk_lvl[s] : q;
     }
-    rv[t] = bv;
-    rc[t] = bc;
-    rl[t] = bl;
-    __syncthreads();
-    if (t == 0) {
-      for (int s = 1; s < (int)blockDim.x; ++s)
-        if (better(rv[s], rc[s], bv, bc)) {
-          bv = rv[s];
-          bc = rc[s];
-          bl = rl[s];
-        }
-      if (q < 0) {
-        out[0] = bc >= 0 ? bv : 0.0;
-        iout[0] = bc;
-        iout[1] = bl;
-      } else {
-        out[1 + q] = bc >= 0 ? bv : 0.0;
-      }
+  }
+  rv[t] = bv;
+  rc[t] = bc;
+  rl[t] = bl;
+  __syncthreads();
+  for (int h = 128; h > 0; h /= 2) {
+    if (t < h && better(rv[t + h], rc[t + h], rv[t], rc[t])) {
+      rv[t] = rv[t + h];
+      rc[t] = rc[t + h];
+      rl[t] = rl[t + h];
     }
     __syncthreads();
+  }
+  if (t == 0) {
+    out[1 + q] = rc[0] >= 0 ? rv[0] : 0.0;
+    if (q < 0) {
+      iout[0] = rc[0];
+      iout[1] = rl[0];
+    }
   }
 }
 
@@ -296,8 +336,8 @@ __global__ void __launch_bounds__(256) normalize_kernel(int nrad, int nline, int
 int rate_solve(m3drt_ctx *ctx, const m3drt_rate_solve_args *r, m3drt_rate_solve_result *res) {
   const int nk = r->nk;
   const size_t per_cell = ((size_t)nk * nk + 2 * (size_t)nk + 2) * sizeof(double) + 2 * sizeof(int);
-  int nt = (int)std::min<size_t>(64, (size_t)ctx->lds_max / per_cell);
-  if (nt >= 8) nt -= nt % 8;
+  int nt = (int)std::min<size_t>(kSeCells, (size_t)ctx->lds_max / per_cell);
+  if (nt >= 4) nt -= nt % 4;
   if (nt < 1) return set_error(M3DRT_ELIMIT, "m3drt_rate_solve_f64: nk too large for the LDS");
   const int nblk = (r->ncell + nt - 1) / nt;
   const size_t lds = per_cell * nt;
@@ -334,9 +374,9 @@ int rate_solve(m3drt_ctx *ctx, const m3drt_rate_solve_args *r, m3drt_rate_solve_
   a.blk_lcell = blk_lcell; a.nclamp = nclamp; a.status = status;
   M3DRT_HIP(hipFuncSetAttribute((const void *)se_update_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)lds));
-  hipLaunchKernelGGL(se_update_kernel, dim3(nblk), dim3(nt), lds, ctx->stream, a);
+  hipLaunchKernelGGL(se_update_kernel, dim3(nblk), dim3(nt * kSeLanes), lds, ctx->stream, a);
   M3DRT_HIP(hipGetLastError());
-  hipLaunchKernelGGL(se_final_kernel, dim3(1), dim3(256), 0, ctx->stream, nblk, nk, blk_err, blk_cell, blk_lvl,
+  hipLaunchKernelGGL(se_final_kernel, dim3(nk + 1), dim3(256), 0, ctx->stream, nblk, nk, blk_err, blk_cell, blk_lvl,
                      blk_lerr, blk_lcell, out, iout);
   M3DRT_HIP(hipGetLastError());
   if (!res) return M3DRT_OK;
