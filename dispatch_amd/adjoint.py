@@ -16,6 +16,11 @@ checkpoint into one patch-sized scratch, and m3drt_sc_adjoint runs the patch in
 reverse, accumulating the cotangents of its chi and S; the cotangent it returns
 for its ghost plane is that of the previous patch's exit plane (I) and last plane
 (chi, S), and is handed on.  Nothing larger than a patch is recomputed or stored.
+
+Where memory allows (a quarter of what is free when the forward pass runs, and J is not
+asked for), a ray's whole intensity cube is kept instead: one sweep of the column writes
+it, one reverse sweep reads it, and the patch by patch recomputation (12 of the 48 B a
+point and ray moves) falls away.  Rays beyond that share are checkpointed.
 The reference has no adjoint; its forward is rt_patch_t%short_char2
 (SRC/rt_solvers_mod.f90:224-507) with integrate_intensity
 (SRC/rt_patch_mod.f90:3399-3431).
@@ -128,6 +133,23 @@ class RaySet:
                 carry = gib.clone()
 
 
+    def adjoint_stored(self, r, chi, S, ghosts, I, gbars, chibar, Sbar, exit_bar=None):
+        """The reverse of the whole column from its intensity cube I."""
+        up = self.up(r)
+        (gc, gs, gi), tb = (ghosts[0], gbars[0]) if up else (ghosts[1], gbars[1])
+        self.ctx.sc_adjoint(chi, S, gc, gs, gi, self.chi500, self.chi500_up[r], self.g500_bot if up else self.g500_top,
+                            I, dir=1 if up else -1, ds=self.ds, vec=self.vec[r], wj=float(self.wj[r]), chibar=chibar,
+                            Sbar=Sbar, exit_bar=exit_bar, ghost_chibar=tb[0], ghost_Sbar=tb[1], ghost_Ibar=tb[2])
+
+
+def _kept_cubes(chi, nray):
+    """How many of nray rays keep their intensity cube: a quarter of the device memory free
+    now (the driver's and the caching allocator's)."""
+    free = torch.cuda.mem_get_info(chi.device)[0]
+    free += torch.cuda.memory_reserved(chi.device) - torch.cuda.memory_allocated(chi.device)
+    return min(nray, free // 4 // max(1, chi.numel() * chi.element_size()))
+
+
 class _FormalSolution(torch.autograd.Function):
     @staticmethod
     def forward(fctx, rs, want_J, rays, chi, S, gc_up, gs_up, gi_up, gc_dn, gs_dn, gi_dn):
@@ -136,11 +158,16 @@ class _FormalSolution(torch.autograd.Function):
         exits = torch.zeros((len(rs.vec), nf, ny, nx), dtype=chi.dtype, device=chi.device)
         J = torch.zeros_like(chi) if want_J else None
         npatch = (nz + rs.patch - 1) // rs.patch
-        ckpt = {}
+        ckpt, cubes = {}, {}
+        keep = 0 if want_J else _kept_cubes(chi, len(rays))
         for r in rays:
+            if len(cubes) < keep and r not in cubes:
+                cubes[r] = torch.empty_like(chi)
+                rs.sweep(r, chi, S, ghosts, I_out=cubes[r], exit_I=exits[r])
+                continue
             ckpt[r] = torch.empty((max(npatch - 1, 1), nf, ny, nx), dtype=chi.dtype, device=chi.device)
             rs.sweep_checkpointed(r, chi, S, ghosts, ckpt[r], exits[r], J=J)
-        fctx.rs, fctx.rays, fctx.ckpt = rs, rays, ckpt
+        fctx.rs, fctx.rays, fctx.ckpt, fctx.cubes = rs, rays, ckpt, cubes
         fctx.save_for_backward(chi, S, gc_up, gs_up, gi_up, gc_dn, gs_dn, gi_dn)
         if want_J:
             return exits, J
@@ -150,7 +177,7 @@ class _FormalSolution(torch.autograd.Function):
 
     @staticmethod
     def backward(fctx, exit_bar, J_bar):
-        rs, rays, ckpt = fctx.rs, fctx.rays, fctx.ckpt
+        rs, rays, ckpt, cubes = fctx.rs, fctx.rays, fctx.ckpt, fctx.cubes
         chi, S, gc_up, gs_up, gi_up, gc_dn, gs_dn, gi_dn = fctx.saved_tensors
         ghosts = ((gc_up, gs_up, gi_up), (gc_dn, gs_dn, gi_dn))
         if J_bar is not None and J_bar.dim() == 0:
@@ -168,13 +195,16 @@ class _FormalSolution(torch.autograd.Function):
         for r in rays:
             if not live[r] and J_bar is None:
                 continue
+            if r in cubes:
+                rs.adjoint_stored(r, chi, S, ghosts, cubes[r], gbars, chibar, Sbar, exit_bar=exit_bar[r])
+                continue
             if scratch is None:
                 scratch = torch.empty((min(rs.patch, chi.shape[0]),) + tuple(chi.shape[1:]), dtype=chi.dtype,
                                       device=chi.device)
                 work = tuple(torch.zeros_like(gc_up) for _ in range(3))
             rs.adjoint_checkpointed(r, chi, S, ghosts, ckpt[r], scratch, gbars, chibar, Sbar, Jbar=J_bar,
                                     exit_bar=exit_bar[r] if live[r] else None, work=work)
-        fctx.ckpt = None
+        fctx.ckpt = fctx.cubes = None
         (gcb_u, gsb_u, gib_u), (gcb_d, gsb_d, gib_d) = gbars
         return None, None, None, chibar, Sbar, gcb_u, gsb_u, gib_u, gcb_d, gsb_d, gib_d
 

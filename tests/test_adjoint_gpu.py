@@ -212,3 +212,34 @@ def test_patch_sweeps_equal_the_column_sweep(ctx):
         assert torch.equal(e1, e2), r
         assert float(e1.abs().max()) > 0
     assert torch.equal(J1, J2)
+
+
+@pytest.mark.parametrize("keep", [1, 3])
+def test_kept_intensities_give_the_checkpointed_gradient(ctx, monkeypatch, keep):
+    """formal_solution keeping the intensity cubes of one of three rays, and of all,
+    against checkpointing every ray: the exit planes bit for bit, the cotangents of chi, S
+    and the ghost planes to the rounding of sums taken in another order (a cell's and a
+    ghost cell's few dozen FP32 terms: 1e-5 of the largest)."""
+    from dispatch_amd import adjoint, synth
+    box = synth.make_box(nx=24, ny=20, nz=30, nf=8, seed=37)
+    chi, S = synth.build_cubes(box, torch.float32)
+    gh = synth.ghost_planes(box, chi, torch.float32)
+    vecs, wj = synth.gauss_rays(6)
+    rs = adjoint.RaySet(ctx, vecs, wj, box.ds, box.chi500, [synth.chi500_upwind(box, v) for v in vecs],
+                        box.g500_bot, box.g500_top, patch=7)
+    rays = [r for r, v in enumerate(vecs) if v[2] > 0][:2] + [r for r, v in enumerate(vecs) if v[2] < 0][:1]
+    g = torch.Generator(device="cuda").manual_seed(2)
+    cot = torch.rand((len(vecs),) + tuple(chi.shape[1:]), generator=g, device="cuda")
+    out = []
+    for n in (0, keep):
+        print(f"kept cubes {n} of {len(rays)}", flush=True)
+        monkeypatch.setattr(adjoint, "_kept_cubes", lambda c, nray, n=n: min(n, nray))
+        leaf = lambda t: t.detach().clone().requires_grad_()
+        c, s = leaf(chi), leaf(S)
+        gu, gd = [leaf(t) for t in gh["up"]], [leaf(t) for t in gh["down"]]
+        exits = adjoint.formal_solution(rs, c, s, gu, gd, rays=rays)
+        exits.backward(cot)
+        out.append([exits.detach(), c.grad, s.grad] + [t.grad for t in gu + gd])
+    assert torch.equal(out[0][0], out[1][0])
+    for k, (a, b) in enumerate(zip(*out)):
+        assert float((a - b).abs().max()) <= 1e-5 * float(a.abs().max()), k
