@@ -66,3 +66,26 @@ def test_rate_solve_lte_fixed_point(ctx):
                        dev(c["gij"], torch.float32), dev(c["gji"], torch.float32), dev(c["cup"], torch.float64))
     assert np.max(np.abs(b.cpu().numpy() - 1.0)) < 1e-5
     assert abs(r["maxerr"]) < 1e-5
+
+
+@pytest.mark.parametrize("nbound,nline,ncont,ncell", [(2, 1, 2, 1), (4, 6, 4, 41), (15, 60, 15, 7), (20, 80, 20, 40),
+                                                     (62, 300, 62, 9), (110, 400, 110, 3)])
+def test_rate_solve_sizes(ctx, monkeypatch, nbound, nline, ncont, ncell):
+    """Level counts below, at and above the sixteen lanes of a cell, workgroups of 40, 4 and
+    1 cells, the last one partly filled: against the oracle as above (1e-10: the rounding of
+    the elimination grows with the level count in both)."""
+    import functools
+    from dispatch_amd import m3drt, synth
+    monkeypatch.setattr(synth, "make_atom", functools.partial(synth.make_atom, nbound=nbound))
+    c = make_se_case(ncell=ncell, seed=ncell, nline=nline, ncont=ncont)
+    print(f"rate solve nbound={nbound} nline={nline} ncell={ncell}", flush=True)
+    bref, rref = O.update_populations(c["atom"], c["e_kT"], c["T"], c["totn"], c["nstar"], c["b"], c["gij"],
+                                      c["gji"], c["cup"])
+    b = dev(c["b"], torch.float64)
+    r = ctx.rate_solve(m3drt.AtomOnDevice(c["atom"]), dev(c["e_kT"], torch.float64), dev(c["T"], torch.float64),
+                       dev(c["totn"], torch.float64), dev(c["nstar"], torch.float64), b,
+                       dev(c["gij"], torch.float32), dev(c["gji"], torch.float32), dev(c["cup"], torch.float64))
+    assert np.max(np.abs(b.cpu().numpy() - bref) / np.abs(bref)) < 1e-10
+    assert (r["epos"], r["elvl"]) == (rref["epos"], rref["elvl"])
+    assert r["nclamp"] == rref["nclamp"]
+    assert np.allclose(r["lvlerr"], rref["lvlerr"], rtol=1e-8, atol=1e-10)
