@@ -41,6 +41,7 @@ struct FastArgs {
   int64_t cs_f, cs_z, gs_f;
   uint32_t cs_x, cs_y, gs_x, gs_y;
   int nx, ny, nz, dir, xo, yo, PW, nstrips;
+  int apart;  // short last strips: the weights rounded as the general kernel's run-time forms do
   uint32_t plane_bytes, gplane_bytes;  // byte reach of one (z, f) plane of a cube / the ghost plane
   T xk0, xk1, xk2, xk3, yk0, yk1, yk2, yk3, hx, hy, mdtau, imax, wj;
 };
@@ -100,6 +101,50 @@ __global__ void __launch_bounds__(256) sc2_prep_pairs(const float *__restrict__ 
     }
     dr[i] = p;
   }
+}
+
+// dev::lin_weights with every rounding written out, for the strips that stand in for
+// another kernel: the upwind intensity's clamp (the larger of the cubic value and the
+// stencil's minimum) takes a last bit for a choice, and an adjoint through that choice
+// sends a whole cotangent elsewhere (gradients moved by 1.5e-3 in norm), so a plane's
+// intensities must not depend on which kernel sweeps it.  The compiler joins products
+// and sums by how often a value is used: where the outputs are fixed and Esc is not
+// among them, W = u0/t - E is one fused step with E rounded; where Esc is formed (SPL),
+// or the general kernel tests its outputs at run time (apart), u0/t is rounded and E is
+// not, and with apart Psi is rounded before Esc = 1 - Psi.
+template <bool SPL>
+__device__ __forceinline__ void lin_weights_as(bool apart, float t, float &E, float &W, float &Psi, float &Esc) {
+#pragma clang fp contract(off)
+  auto fma = [](float a, float b, float c) { return __builtin_fmaf(a, b, c); };
+  float P = fma(t, -2.834696488e-06f, 2.522676368e-05f);
+  P = fma(t, P, -1.983609400e-04f);
+  P = fma(t, P, 1.388740959e-03f);
+  P = fma(t, P, -8.333330974e-03f);
+  P = fma(t, P, 4.166666791e-02f);
+  P = fma(t, P, -1.666666716e-01f);
+  P = fma(t, P, 5.000000000e-01f);
+  const float ps = t * P;
+  // exp_neg
+  const float tc = fminf(t, 87.0f);
+  const float n = __builtin_rintf(tc * 1.44269504088896341f);
+  float r = fma(-n, 0.693359375f, tc);
+  r = fma(-n, -2.12194440e-4f, r);
+  float M = fma(r, -2.48015876e-05f, 1.98412701e-04f);
+  M = fma(r, M, -1.38888892e-03f);
+  M = fma(r, M, 8.33333377e-03f);
+  M = fma(r, M, -4.16666679e-02f);
+  M = fma(r, M, 1.66666672e-01f);
+  M = fma(r, M, -0.5f);
+  M = fma(r, M, 1.0f);
+  const float q = fma(-r, M, 1.0f), s = __builtin_ldexpf(1.0f, -(int)n);
+  const float u0 = fma(s, r * M, 1.0f - s);
+  E = s * q;
+  const float rt = dev::rcp(t), ut = u0 * rt;
+  const bool thin = fabsf(t) <= 1.0f;
+  Psi = thin ? ps : fma(-rt, u0, 1.0f);
+  const float far = SPL || apart ? fma(-s, q, ut) : fma(rt, u0, -E);
+  W = thin ? fma(-t, P, u0) : far;
+  Esc = thin ? (apart ? 1.0f - ps : fma(-t, P, 1.0f)) : ut;
 }
 
 template <typename T, int N>
@@ -329,7 +374,8 @@ __global__ void __launch_bounds__(fast_max_threads<L>()) sc2_fast(const FastArgs
         T dt = (T)0.5 * (xxup + xx) * dt500;
         dt = fmax(dt, a.mdtau);
         T E, W, Ps, Es;
-        lin_weights(dt, E, W, Ps, Es);
+        if (RAG) lin_weights_as<SPL>(a.apart, dt, E, W, Ps, Es);
+        else lin_weights(dt, E, W, Ps, Es);
         // the S step of a cell without eta flags (SRC/rt_solvers_mod.f90:419-440, 465-475)
         const T Ir = Inuup * E + W * ssup;
         T Inu = Ir + Ps * ss;
@@ -661,6 +707,9 @@ int run_fast(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const m3drt_sweep_bufs *
   const int64_t pts = (int64_t)nx * ny * d->nf;
   const bool rag = Lr && (!L || rwant || (Lr < L && d->nf >= 8 && pts < (L == 4 ? 180000 : 1300000)) ||
                           (L == 4 && Lr > 4 && ny / 4 * nx > 512));
+  // the kernel that would take the call without them: the general one (strips of 24 and
+  // 30 have no per-cell outputs), or strips that divide ny
+  const bool general = !L || ((spl || iout) && L > 20);
   if (rag) L = Lr;
   if (!L) return -1;
   const int nstrips = (ny + L - 1) / L;
@@ -721,6 +770,7 @@ int run_fast(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const m3drt_sweep_bufs *
   a.gs_x = (uint32_t)d->gs_x; a.gs_y = (uint32_t)d->gs_y;
   a.nx = nx; a.ny = ny; a.nz = nz; a.dir = d->dir > 0 ? 1 : -1;
   a.xo = g.xo; a.yo = g.yo; a.PW = nx + 4; a.nstrips = nstrips;
+  a.apart = general && !sc2_general_fixed_outputs(d, b);
   a.plane_bytes = (uint32_t)((span + 1) * sizeof(T));
   a.gplane_bytes = (uint32_t)((gspan + 1) * sizeof(T));
   // the stencil in FP32 as the reference casts it (FP64 sweep: in FP64)

@@ -458,6 +458,29 @@ static int sc2_limits(m3drt_ctx *ctx, const m3drt_sweep_desc *d) {
   return M3DRT_OK;
 }
 
+// The strip length of the straight-line form that the general kernel takes, 0 if none:
+// where only J (and PsiJ), or only the intensity cube, are asked for, or (any_out; FP32,
+// strips of at most 12 rows) any outputs but the eta step, checked at run time, and an
+// instantiated length of at least L rows divides ny.
+template <typename T>
+static int exact_strip(const m3drt_sweep_desc *d, const m3drt_sweep_bufs *b, int L, bool &any_out) {
+  const bool psi_out = (d->flags & M3DRT_GET_RATES) && (b->Psi_out || b->PsiJ);
+  const bool plain_out = !b->eta_row && !(d->flags & M3DRT_SPLIT_RATES) &&
+                         ((!b->I_out && b->J && !((d->flags & M3DRT_GET_RATES) && b->Psi_out)) ||
+                          (b->I_out && !b->J && !psi_out));
+  any_out = !plain_out && !b->eta_row && sizeof(T) == 4;
+  if ((plain_out || any_out) && !getenv("M3DRT_NO_EXACT"))
+    for (int c : (sizeof(T) == 4 ? kExactL32 : kExactL64))
+      if (c >= L && d->ny % c == 0 && !(any_out && c > 12)) return c;
+  return 0;
+}
+
+bool sc2_general_fixed_outputs(const m3drt_sweep_desc *d, const m3drt_sweep_bufs *b) {
+  const int smax = std::max(1, 1024 / d->nx);
+  bool any_out;
+  return exact_strip<float>(d, b, (d->ny + smax - 1) / smax, any_out) && !any_out;
+}
+
 template <typename T>
 static int run_sc2(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const m3drt_sweep_bufs *b) {
   const int nx = d->nx, ny = d->ny, nz = d->nz;
@@ -469,20 +492,8 @@ static int run_sc2(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const m3drt_sweep_
   const int tmax = sizeof(T) == 8 ? 512 : 1024;
   const int smax = std::max(1, tmax / nx);
   int L = (ny + smax - 1) / smax;
-  // the straight-line form when only J (and PsiJ), or only the intensity cube, are
-  // asked for and an instantiated strip length divides ny
-  int Lexact = 0;
-  const bool psi_out = (d->flags & M3DRT_GET_RATES) && (b->Psi_out || b->PsiJ);
-  const bool plain_out = !b->eta_row && !(d->flags & M3DRT_SPLIT_RATES) &&
-                         ((!b->I_out && b->J && !((d->flags & M3DRT_GET_RATES) && b->Psi_out)) ||
-                          (b->I_out && !b->J && !psi_out));
-  // FP32 with any other outputs but the eta step (the ALI's I, Psi, Irem, escape): the
-  // exact strips with run-time output checks
-  const bool any_out = !plain_out && !b->eta_row && sizeof(T) == 4;
-  if ((plain_out || any_out) && !getenv("M3DRT_NO_EXACT")) {
-    for (int c : (sizeof(T) == 4 ? kExactL32 : kExactL64))
-      if (c >= L && ny % c == 0 && !Lexact && !(any_out && c > 12)) Lexact = c;
-  }
+  bool any_out;
+  const int Lexact = exact_strip<T>(d, b, L, any_out);
   if (Lexact) L = Lexact;
   const int nstrips = (ny + L - 1) / L;
   const int nt = nx * nstrips;

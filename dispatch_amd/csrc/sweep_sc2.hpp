@@ -49,6 +49,10 @@ int sc2_prep(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const float *chi500, con
 template <typename T>
 int sweep_sc2_plane(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const m3drt_sweep_bufs *b);
 
+// Whether the general FP32 kernel would take this call in a form whose outputs are fixed
+// at compile time: its far weights then round as sc2_fast's, else apart (sc2_fast.hip).
+bool sc2_general_fixed_outputs(const m3drt_sweep_desc *d, const m3drt_sweep_bufs *b);
+
 // The straight-line sweep for J (and PsiJ) only; returns -1 when the case is not
 // one it takes (the caller then runs the general kernel), else a status.
 int sweep_sc2_fast(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const m3drt_sweep_bufs *b);

@@ -476,3 +476,37 @@ def test_sweep_short_last_strip_matches_oracle(ctx, monkeypatch, rows, nx, ny, n
         for k, t in o.items():
             check32(back(t), ref[k], f"{k} of {outs}")
         check32(np.moveaxis(ex.double().cpu().numpy(), 0, 2), I[last], f"exit plane of {outs}")
+
+
+# the kernel that sweeps a plane does not show in its values: the strips with a short last
+# one give the bits of the kernel they stand in for -- the general one with outputs tested
+# at run time (exit plane alone; no strip divides ny), the general one with fixed outputs
+# (one strip of 12 or 15), and the strips that divide ny (few points) -- for S in LDS and
+# from the cache, and the general kernel's strips of up to 4, 8, 16 and 32 rows
+@pytest.mark.parametrize("nf,nx,ny,nz", [
+    (20, 101, 67, 6), (33, 9, 13, 8), (8, 120, 119, 4), (8, 117, 113, 4), (250, 40, 41, 5), (40, 16, 61, 6),
+    (12, 5, 7, 9), (6, 60, 15, 5), (9, 250, 12, 4), (9, 48, 48, 6), (64, 12, 30, 6), (16, 110, 75, 4), (7, 17, 701, 3),
+    (10, 90, 144, 3),
+])
+def test_short_last_strips_keep_the_bits(ctx, monkeypatch, nf, nx, ny, nz):
+    g = torch.Generator(device="cuda").manual_seed(nx * ny)
+    r = lambda *s: torch.rand(s, generator=g, device="cuda") + 0.5
+    chi = r(nz, nf, ny, nx) * 1e-7 * torch.logspace(1, -2.5, nz, device="cuda")[:, None, None, None]
+    S, gh = r(nz, nf, ny, nx), [r(nf, ny, nx) * 1e-6, r(nf, ny, nx), r(nf, ny, nx)]
+    c5, cu, g5 = r(nz, ny, nx) * 1e-7, r(nz, ny, nx) * 1e-7, r(ny, nx) * 1e-7
+    rates = dict(get_rates=True)
+    for outs, kw in (((), {}), (("I_out",), {}), (("J",), {}), (("J", "PsiJ"), rates),
+                     (("I_out", "Psi_out", "Irem_out", "escape_out"), dict(rates, split_rates=True))):
+        got = []
+        for norag in (True, False):
+            if norag:
+                monkeypatch.setenv("M3DRT_NO_RAG", "1")
+            else:
+                monkeypatch.delenv("M3DRT_NO_RAG")
+            o = {k: torch.full_like(chi, 0.125) for k in outs}
+            ex = torch.zeros_like(gh[0])
+            ctx.sc_sweep(chi, S, *gh, c5, cu, g5, dir=1, ds=(50e5, 50e5, 10e5), vec=(0.3, -0.4, 0.866), wj=0.25,
+                         exit_I=ex, **kw, **o)
+            got.append(dict(o, exit=ex))
+        for k in got[0]:
+            assert torch.equal(got[0][k], got[1][k]), (outs, k)
