@@ -526,15 +526,17 @@ template <int L, int CPL>
 int fast_variant(m3drt_ctx *ctx, const FastArgs<float> &a, int nf, int nt, int mode, size_t np, int sr) {
   const size_t l2 = np * 2 * sizeof(float), l3 = np * 3 * sizeof(float);
   const size_t l4 = l2 + (size_t)(a.nstrips * sr + 1) * a.nx * sizeof(float);
-  if (a.Iout) {  // per-cell outputs (the split set, or I alone), for the strip lengths 4 to 20
+  if (a.Psiout) {  // the split set, for the strip lengths 4 to 20
     if constexpr (CPL == 1 && (L == 4 || L == 12 || L == 15 || L == 20)) {
-      if (a.Psiout) {
-        if (mode == 2) return launch_fast<L, false, 2, CPL, 0, 1>(ctx, a, nf, nt, l3);
-        if (mode == 1) return launch_fast<L, false, 1, CPL, 0, 1>(ctx, a, nf, nt, l2);
-      } else {
-        if (mode == 2) return launch_fast<L, false, 2, CPL, 0, 2>(ctx, a, nf, nt, l3);
-        if (mode == 1) return launch_fast<L, false, 1, CPL, 0, 2>(ctx, a, nf, nt, l2);
-      }
+      if (mode == 2) return launch_fast<L, false, 2, CPL, 0, 1>(ctx, a, nf, nt, l3);
+      if (mode == 1) return launch_fast<L, false, 1, CPL, 0, 1>(ctx, a, nf, nt, l2);
+    }
+    return -1;
+  }
+  if (a.Iout) {  // I alone: wherever the exit plane alone is taken, with the same values
+    if constexpr (CPL == 1) {
+      if (mode == 2) return launch_fast<L, false, 2, CPL, 0, 2>(ctx, a, nf, nt, l3);
+      if (mode == 1) return launch_fast<L, false, 1, CPL, 0, 2>(ctx, a, nf, nt, l2);
     }
     return -1;
   }
@@ -708,8 +710,8 @@ int run_fast(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const m3drt_sweep_bufs *
   const bool rag = Lr && (!L || rwant || (Lr < L && d->nf >= 8 && pts < (L == 4 ? 180000 : 1300000)) ||
                           (L == 4 && Lr > 4 && ny / 4 * nx > 512));
   // the kernel that would take the call without them: the general one (strips of 24 and
-  // 30 have no per-cell outputs), or strips that divide ny
-  const bool general = !L || ((spl || iout) && L > 20);
+  // 30 have no split outputs), or strips that divide ny
+  const bool general = !L || (spl && L > 20);
   if (rag) L = Lr;
   if (!L) return -1;
   const int nstrips = (ny + L - 1) / L;

@@ -459,15 +459,16 @@ static int sc2_limits(m3drt_ctx *ctx, const m3drt_sweep_desc *d) {
 }
 
 // The strip length of the straight-line form that the general kernel takes, 0 if none:
-// where only J (and PsiJ), or only the intensity cube, are asked for, or (any_out; FP32,
-// strips of at most 12 rows) any outputs but the eta step, checked at run time, and an
-// instantiated length of at least L rows divides ny.
+// where only J (and PsiJ), or only the intensity cube (in FP32 also only the exit plane,
+// so that its values are the cube's: an adjoint mixes the two), are asked for, or
+// (any_out; FP32, strips of at most 12 rows) any outputs but the eta step, checked at run
+// time, and an instantiated length of at least L rows divides ny.
 template <typename T>
 static int exact_strip(const m3drt_sweep_desc *d, const m3drt_sweep_bufs *b, int L, bool &any_out) {
   const bool psi_out = (d->flags & M3DRT_GET_RATES) && (b->Psi_out || b->PsiJ);
   const bool plain_out = !b->eta_row && !(d->flags & M3DRT_SPLIT_RATES) &&
                          ((!b->I_out && b->J && !((d->flags & M3DRT_GET_RATES) && b->Psi_out)) ||
-                          (b->I_out && !b->J && !psi_out));
+                          ((b->I_out || sizeof(T) == 4) && !b->J && !psi_out));
   any_out = !plain_out && !b->eta_row && sizeof(T) == 4;
   if ((plain_out || any_out) && !getenv("M3DRT_NO_EXACT"))
     for (int c : (sizeof(T) == 4 ? kExactL32 : kExactL64))

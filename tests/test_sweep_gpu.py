@@ -510,3 +510,25 @@ def test_short_last_strips_keep_the_bits(ctx, monkeypatch, nf, nx, ny, nz):
             got.append(dict(o, exit=ex))
         for k in got[0]:
             assert torch.equal(got[0][k], got[1][k]), (outs, k)
+
+
+# an adjoint takes its checkpoints from sweeps of the exit plane alone and recomputes
+# (or keeps) the intensities between them: the two have the same bits whichever kernels
+# the plane takes -- strips of every length, a single strip, no straight-line form at all
+@pytest.mark.parametrize("nf,nx,ny,nz", [
+    (9, 24, 20, 4), (5, 131, 96, 3), (120, 131, 96, 3), (6, 130, 120, 3), (4, 120, 120, 3), (4, 96, 96, 3), (6, 60, 15, 4),
+    (5, 400, 12, 3), (8, 9, 4, 5), (8, 3, 4, 5), (8, 4, 3, 5), (8, 30, 5, 4), (4, 101, 67, 3), (3, 119, 105, 3), (4, 60, 60, 4),
+])
+def test_exit_plane_alone_has_the_cubes_bits(ctx, nf, nx, ny, nz):
+    g = torch.Generator(device="cuda").manual_seed(nx + ny)
+    r = lambda *s: torch.rand(s, generator=g, device="cuda") + 0.5
+    chi = r(nz, nf, ny, nx) * 1e-7 * torch.logspace(1, -2.5, nz, device="cuda")[:, None, None, None]
+    S, gh = r(nz, nf, ny, nx), [r(nf, ny, nx) * 1e-6, r(nf, ny, nx), r(nf, ny, nx)]
+    c5, cu, g5 = r(nz, ny, nx) * 1e-7, r(nz, ny, nx) * 1e-7, r(ny, nx) * 1e-7
+    geo = dict(dir=1, ds=(50e5, 50e5, 10e5), vec=(0.3, -0.4, 0.866))
+    I, alone, beside = torch.zeros_like(chi), torch.zeros_like(gh[0]), torch.zeros_like(gh[0])
+    ctx.sc_sweep(chi, S, *gh, c5, cu, g5, exit_I=alone, **geo)
+    ctx.sc_sweep(chi, S, *gh, c5, cu, g5, exit_I=beside, I_out=I, **geo)
+    assert float(alone.abs().max()) > 0
+    assert torch.equal(beside, I[-1])
+    assert torch.equal(alone, beside), float((alone - beside).abs().max())
