@@ -15,12 +15,12 @@ taken in reverse sweep order: the patch's intensity is recomputed from its
 checkpoint into one patch-sized scratch, and m3drt_sc_adjoint runs the patch in
 reverse, accumulating the cotangents of its chi and S; the cotangent it returns
 for its ghost plane is that of the previous patch's exit plane (I) and last plane
-(chi, S), and is handed on.  Nothing larger than a patch is recomputed or stored.
+(chi, S), and is handed on.  Nothing larger than a patch is recomputed.
 
 Where memory allows (a quarter of what is free when the forward pass runs, and J is not
-asked for), a ray's whole intensity cube is kept instead: one sweep of the column writes
-it, one reverse sweep reads it, and the patch by patch recomputation (12 of the 48 B a
-point and ray moves) falls away.  Rays beyond that share are checkpointed.
+asked for), the forward also keeps a ray's whole intensity cube, and the recomputation
+(12 of the 48 B a point and ray moves) falls away.  The patches are the same either way,
+and so is every sum's order: what is kept changes the time, not a bit of the gradient.
 The reference has no adjoint; its forward is rt_patch_t%short_char2
 (SRC/rt_solvers_mod.f90:224-507) with integrate_intensity
 (SRC/rt_patch_mod.f90:3399-3431).
@@ -90,56 +90,53 @@ class RaySet:
         self.ctx.sc_sweep(chi[z0:z1], S[z0:z1], gc, gs, gi, self.chi500[z0:z1], self.chi500_up[r][z0:z1], g500,
                           dir=1 if self.up(r) else -1, ds=self.ds, vec=self.vec[r], wj=float(self.wj[r]), **out)
 
-    def sweep_checkpointed(self, r, chi, S, ghosts, ckpt, exit_I, J=None):
+    def sweep_checkpointed(self, r, chi, S, ghosts, ckpt, exit_I, J=None, cube=None):
         """The ray patch by patch: ckpt (npatch - 1, nf, ny, nx) receives the exit
-        plane of every patch but the last, whose exit plane goes to exit_I."""
+        plane of every patch but the last, whose exit plane goes to exit_I; cube, if
+        given, every cell's intensity."""
         bounds = self.patches(r, chi.shape[0])
-        for k in range(len(bounds)):
+        for k, (z0, z1) in enumerate(bounds):
             ex = ckpt[k] if k + 1 < len(bounds) else exit_I
-            self.sweep_patch(r, k, bounds, chi, S, ghosts, ckpt, exit_I=ex, J=J)
+            out = {} if cube is None else {"I_out": cube[z0:z1]}
+            self.sweep_patch(r, k, bounds, chi, S, ghosts, ckpt, exit_I=ex, J=J, **out)
 
     def adjoint_checkpointed(self, r, chi, S, ghosts, ckpt, scratch, gbars, chibar, Sbar, Jbar=None,
-                             exit_bar=None, work=None):
+                             exit_bar=None, work=None, cube=None):
         """The reverse of sweep_checkpointed: patch by patch from the exit, each
-        patch's intensity recomputed from its checkpoint into scratch (>= patch
-        planes).  gbars: the true ghost planes' cotangents (accumulated); work: three
+        patch's intensity read from cube, or recomputed from its checkpoint into scratch
+        (>= patch planes).  gbars: the true ghost planes' cotangents (accumulated); work: three
         (nf, ny, nx) planes for the patch-boundary cotangents."""
         bounds = self.patches(r, chi.shape[0])
         up = self.up(r)
-        gcb, gsb, gib = work
+        gcb, *gib = work
         carry = exit_bar
         for k in range(len(bounds) - 1, -1, -1):
             z0, z1 = bounds[k]
-            n = z1 - z0
-            I = scratch[:n]
-            self.sweep_patch(r, k, bounds, chi, S, ghosts, ckpt, I_out=I)
+            if cube is not None:
+                I = cube[z0:z1]
+            else:
+                I = scratch[:z1 - z0]
+                self.sweep_patch(r, k, bounds, chi, S, ghosts, ckpt, I_out=I)
             (gc, gs, gi), g500 = self._ghost_of(r, k, bounds, chi, S, ghosts, ckpt)
             if k == 0:
                 tb = gbars[0] if up else gbars[1]
                 ghost_bars = dict(ghost_chibar=tb[0], ghost_Sbar=tb[1], ghost_Ibar=tb[2])
             else:
-                for t in work:
-                    t.zero_()
-                ghost_bars = dict(ghost_chibar=gcb, ghost_Sbar=gsb, ghost_Ibar=gib)
+                # the previous patch's last plane: S's cotangent added in place, chi's
+                # product rounded before it is added, I's in the plane not read now
+                pz0, pz1 = bounds[k - 1]
+                zl = pz1 - 1 if up else pz0
+                below = gib[k % 2]
+                gcb.zero_()
+                below.zero_()
+                ghost_bars = dict(ghost_chibar=gcb, ghost_Sbar=Sbar[zl], ghost_Ibar=below)
             self.ctx.sc_adjoint(chi[z0:z1], S[z0:z1], gc, gs, gi, self.chi500[z0:z1], self.chi500_up[r][z0:z1],
                                 g500, I, dir=1 if up else -1, ds=self.ds, vec=self.vec[r], wj=float(self.wj[r]),
                                 chibar=chibar[z0:z1], Sbar=Sbar[z0:z1],
                                 Jbar=None if Jbar is None else Jbar[z0:z1], exit_bar=carry, **ghost_bars)
             if k > 0:
-                pz0, pz1 = bounds[k - 1]
-                zl = pz1 - 1 if up else pz0
                 chibar[zl] += gcb
-                Sbar[zl] += gsb
-                carry = gib.clone()
-
-
-    def adjoint_stored(self, r, chi, S, ghosts, I, gbars, chibar, Sbar, exit_bar=None):
-        """The reverse of the whole column from its intensity cube I."""
-        up = self.up(r)
-        (gc, gs, gi), tb = (ghosts[0], gbars[0]) if up else (ghosts[1], gbars[1])
-        self.ctx.sc_adjoint(chi, S, gc, gs, gi, self.chi500, self.chi500_up[r], self.g500_bot if up else self.g500_top,
-                            I, dir=1 if up else -1, ds=self.ds, vec=self.vec[r], wj=float(self.wj[r]), chibar=chibar,
-                            Sbar=Sbar, exit_bar=exit_bar, ghost_chibar=tb[0], ghost_Sbar=tb[1], ghost_Ibar=tb[2])
+                carry = below
 
 
 def _kept_cubes(chi, nray):
@@ -161,12 +158,10 @@ class _FormalSolution(torch.autograd.Function):
         ckpt, cubes = {}, {}
         keep = 0 if want_J else _kept_cubes(chi, len(rays))
         for r in rays:
+            ckpt[r] = torch.empty((max(npatch - 1, 1), nf, ny, nx), dtype=chi.dtype, device=chi.device)
             if len(cubes) < keep and r not in cubes:
                 cubes[r] = torch.empty_like(chi)
-                rs.sweep(r, chi, S, ghosts, I_out=cubes[r], exit_I=exits[r])
-                continue
-            ckpt[r] = torch.empty((max(npatch - 1, 1), nf, ny, nx), dtype=chi.dtype, device=chi.device)
-            rs.sweep_checkpointed(r, chi, S, ghosts, ckpt[r], exits[r], J=J)
+            rs.sweep_checkpointed(r, chi, S, ghosts, ckpt[r], exits[r], J=J, cube=cubes.get(r))
         fctx.rs, fctx.rays, fctx.ckpt, fctx.cubes = rs, rays, ckpt, cubes
         fctx.save_for_backward(chi, S, gc_up, gs_up, gi_up, gc_dn, gs_dn, gi_dn)
         if want_J:
@@ -195,15 +190,13 @@ class _FormalSolution(torch.autograd.Function):
         for r in rays:
             if not live[r] and J_bar is None:
                 continue
-            if r in cubes:
-                rs.adjoint_stored(r, chi, S, ghosts, cubes[r], gbars, chibar, Sbar, exit_bar=exit_bar[r])
-                continue
-            if scratch is None:
+            if scratch is None and r not in cubes:
                 scratch = torch.empty((min(rs.patch, chi.shape[0]),) + tuple(chi.shape[1:]), dtype=chi.dtype,
                                       device=chi.device)
+            if work is None:
                 work = tuple(torch.zeros_like(gc_up) for _ in range(3))
             rs.adjoint_checkpointed(r, chi, S, ghosts, ckpt[r], scratch, gbars, chibar, Sbar, Jbar=J_bar,
-                                    exit_bar=exit_bar[r] if live[r] else None, work=work)
+                                    exit_bar=exit_bar[r] if live[r] else None, work=work, cube=cubes.get(r))
         fctx.ckpt = fctx.cubes = None
         (gcb_u, gsb_u, gib_u), (gcb_d, gsb_d, gib_d) = gbars
         return None, None, None, chibar, Sbar, gcb_u, gsb_u, gib_u, gcb_d, gsb_d, gib_d

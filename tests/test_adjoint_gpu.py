@@ -243,3 +243,32 @@ def test_kept_intensities_give_the_checkpointed_gradient(ctx, monkeypatch, keep)
     assert torch.equal(out[0][0], out[1][0])
     for k, (a, b) in enumerate(zip(*out)):
         assert float((a - b).abs().max()) <= 1e-5 * float(a.abs().max()), k
+
+
+@pytest.mark.parametrize("nx,ny,nz,nf,patch", [(24, 20, 30, 8, 7), (29, 33, 17, 12, 5), (16, 15, 12, 9, 4), (40, 17, 9, 43, 23)])
+def test_kept_intensities_do_not_change_the_bits(ctx, monkeypatch, nx, ny, nz, nf, patch):
+    """How many rays keep their cubes depends on the memory that is free: the exit planes
+    and every cotangent are the same bits for none, one and all of three rays kept, on
+    planes that strips divide and others, with whole and cut patches."""
+    from dispatch_amd import adjoint, synth
+    box = synth.make_box(nx=nx, ny=ny, nz=nz, nf=nf, seed=nx + ny)
+    chi, S = synth.build_cubes(box, torch.float32)
+    gh = synth.ghost_planes(box, chi, torch.float32)
+    vecs, wj = synth.gauss_rays(6)
+    rs = adjoint.RaySet(ctx, vecs, wj, box.ds, box.chi500, [synth.chi500_upwind(box, v) for v in vecs],
+                        box.g500_bot, box.g500_top, patch=patch)
+    rays = [r for r, v in enumerate(vecs) if v[2] > 0][:2] + [r for r, v in enumerate(vecs) if v[2] < 0][:1]
+    g = torch.Generator(device="cuda").manual_seed(2)
+    cot = torch.rand((len(vecs),) + tuple(chi.shape[1:]), generator=g, device="cuda")
+    out = []
+    for n in (0, 1, 3):
+        monkeypatch.setattr(adjoint, "_kept_cubes", lambda c, nray, n=n: min(n, nray))
+        leaf = lambda t: t.detach().clone().requires_grad_()
+        c, s = leaf(chi), leaf(S)
+        gu, gd = [leaf(t) for t in gh["up"]], [leaf(t) for t in gh["down"]]
+        exits = adjoint.formal_solution(rs, c, s, gu, gd, rays=rays)
+        exits.backward(cot)
+        out.append([exits.detach(), c.grad, s.grad] + [t.grad for t in gu + gd])
+    assert float(out[0][1].abs().max()) > 0
+    for k, (a, b, c) in enumerate(zip(*out)):
+        assert torch.equal(a, b) and torch.equal(a, c), k
