@@ -17,8 +17,8 @@ reverse, accumulating the cotangents of its chi and S; the cotangent it returns
 for its ghost plane is that of the previous patch's exit plane (I) and last plane
 (chi, S), and is handed on.  Nothing larger than a patch is recomputed.
 
-Where memory allows (a quarter of what is free when the forward pass runs, and J is not
-asked for), the forward also keeps a ray's whole intensity cube, and the recomputation
+Where memory allows (a quarter of what is free when the forward pass runs), a gradient
+will be taken and J is not asked for, the forward also keeps a ray's whole intensity cube, and the recomputation
 (12 of the 48 B a point and ray moves) falls away.  The patches are the same either way,
 and so is every sum's order: what is kept changes the time, not a bit of the gradient.
 The reference has no adjoint; its forward is rt_patch_t%short_char2
@@ -149,14 +149,14 @@ def _kept_cubes(chi, nray):
 
 class _FormalSolution(torch.autograd.Function):
     @staticmethod
-    def forward(fctx, rs, want_J, rays, chi, S, gc_up, gs_up, gi_up, gc_dn, gs_dn, gi_dn):
+    def forward(fctx, rs, want_J, rays, grad, chi, S, gc_up, gs_up, gi_up, gc_dn, gs_dn, gi_dn):
         ghosts = ((gc_up, gs_up, gi_up), (gc_dn, gs_dn, gi_dn))
         nz, nf, ny, nx = chi.shape
         exits = torch.zeros((len(rs.vec), nf, ny, nx), dtype=chi.dtype, device=chi.device)
         J = torch.zeros_like(chi) if want_J else None
         npatch = (nz + rs.patch - 1) // rs.patch
         ckpt, cubes = {}, {}
-        keep = 0 if want_J else _kept_cubes(chi, len(rays))
+        keep = _kept_cubes(chi, len(rays)) if grad and not want_J else 0
         for r in rays:
             ckpt[r] = torch.empty((max(npatch - 1, 1), nf, ny, nx), dtype=chi.dtype, device=chi.device)
             if len(cubes) < keep and r not in cubes:
@@ -199,7 +199,7 @@ class _FormalSolution(torch.autograd.Function):
                                     exit_bar=exit_bar[r] if live[r] else None, work=work, cube=cubes.get(r))
         fctx.ckpt = fctx.cubes = None
         (gcb_u, gsb_u, gib_u), (gcb_d, gsb_d, gib_d) = gbars
-        return None, None, None, chibar, Sbar, gcb_u, gsb_u, gib_u, gcb_d, gsb_d, gib_d
+        return None, None, None, None, chibar, Sbar, gcb_u, gsb_u, gib_u, gcb_d, gsb_d, gib_d
 
 
 def formal_solution(rs: RaySet, chi, S, ghost_up, ghost_down, want_J=False, rays=None):
@@ -210,5 +210,6 @@ def formal_solution(rs: RaySet, chi, S, ghost_up, ghost_down, want_J=False, rays
     the rays to sweep (default all; the others' exit planes stay zero and they add
     nothing to J)."""
     rays = list(range(len(rs.vec))) if rays is None else [int(r) for r in rays]
-    exits, J = _FormalSolution.apply(rs, want_J, rays, chi, S, *ghost_up, *ghost_down)
+    grad = torch.is_grad_enabled() and any(t.requires_grad for t in (chi, S, *ghost_up, *ghost_down))
+    exits, J = _FormalSolution.apply(rs, want_J, rays, grad, chi, S, *ghost_up, *ghost_down)
     return (exits, J) if want_J else exits

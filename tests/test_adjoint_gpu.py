@@ -272,3 +272,25 @@ def test_kept_intensities_do_not_change_the_bits(ctx, monkeypatch, nx, ny, nz, n
     assert float(out[0][1].abs().max()) > 0
     for k, (a, b, c) in enumerate(zip(*out)):
         assert torch.equal(a, b) and torch.equal(a, c), k
+
+
+def test_nothing_is_kept_without_a_gradient(ctx, monkeypatch):
+    """Under no_grad, and with no input that needs a gradient, no intensity cube is
+    written: the exit planes are the same bits as those of a differentiated call."""
+    from dispatch_amd import adjoint, synth
+    box = synth.make_box(nx=12, ny=10, nz=9, nf=6, seed=3)
+    chi, S = synth.build_cubes(box, torch.float32)
+    gh = synth.ghost_planes(box, chi, torch.float32)
+    vecs, wj = synth.gauss_rays(2)
+    rs = adjoint.RaySet(ctx, vecs, wj, box.ds, box.chi500, [synth.chi500_upwind(box, v) for v in vecs],
+                        box.g500_bot, box.g500_top, patch=4)
+    asked = []
+    monkeypatch.setattr(adjoint, "_kept_cubes", lambda c, nray: asked.append(nray) or nray)
+    leaf = chi.clone().requires_grad_()
+    ref = adjoint.formal_solution(rs, leaf, S, gh["up"], gh["down"])
+    assert asked == [len(vecs)]
+    with torch.no_grad():
+        a = adjoint.formal_solution(rs, leaf, S, gh["up"], gh["down"])
+    b = adjoint.formal_solution(rs, chi, S, gh["up"], gh["down"])
+    assert asked == [len(vecs)] and not a.requires_grad and not b.requires_grad
+    assert torch.equal(a, ref) and torch.equal(b, ref)
