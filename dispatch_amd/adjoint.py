@@ -17,10 +17,12 @@ reverse, accumulating the cotangents of its chi and S; the cotangent it returns
 for its ghost plane is that of the previous patch's exit plane (I) and last plane
 (chi, S), and is handed on.  Nothing larger than a patch is recomputed.
 
-Where memory allows (a quarter of what is free when the forward pass runs), a gradient
-will be taken and J is not asked for, the forward also keeps a ray's whole intensity cube, and the recomputation
-(12 of the 48 B a point and ray moves) falls away.  The patches are the same either way,
-and so is every sum's order: what is kept changes the time, not a bit of the gradient.
+Where memory allows, a gradient will be taken and J is not asked for, the forward also
+keeps a ray's whole intensity cube (RaySet.keep), and the recomputation (12 of the 48 B a
+point and ray moves) falls away.  The checkpoints are written all the same, the patches
+are the same either way, and so is every sum's order: a cube is only a shortcut, what is
+kept changes the time and not a bit of the gradient, and cubes are given back wherever an
+allocation here fails or a later solution finds the memory short.
 The reference has no adjoint; its forward is rt_patch_t%short_char2
 (SRC/rt_solvers_mod.f90:224-507) with integrate_intensity
 (SRC/rt_patch_mod.f90:3399-3431).
@@ -29,6 +31,9 @@ chi500 (the tau500 step scale) and the directions are held fixed.
 """
 from __future__ import annotations
 
+import itertools
+import threading
+import weakref
 from dataclasses import dataclass
 
 import numpy as np
@@ -43,7 +48,10 @@ class RaySet:
     (nz, nf, ny, nx): unit vectors (nray, 3), J weights (nray), chi500 (nz, ny, nx),
     chi500 at each ray's upwind points (list of (nz, ny, nx)), the ghost planes'
     chi500 below the bottom and above the top, the cell sizes; `patch` planes per
-    patch of the checkpointed sweep."""
+    patch of the checkpointed sweep; `keep`, how many rays of a solution keep their
+    intensity cubes from the forward to the backward pass at most: a number (0: none, the
+    least memory), or "auto", as many as half of the memory holds that the backward
+    pass and the caller's leave (_kept_cubes).  The results are the same."""
     ctx: "m3drt.Context"
     vec: np.ndarray
     wj: np.ndarray
@@ -53,6 +61,11 @@ class RaySet:
     g500_bot: torch.Tensor
     g500_top: torch.Tensor
     patch: int = 23
+    keep: "int | str" = "auto"
+
+    def __post_init__(self):
+        if self.keep != "auto" and not (isinstance(self.keep, int) and self.keep >= 0):
+            raise ValueError("RaySet.keep is a number of rays or 'auto'")
 
     def up(self, r):
         return self.vec[r][2] > 0
@@ -139,12 +152,78 @@ class RaySet:
                 carry = below
 
 
+class _Cubes:
+    """The intensity cubes that one solution keeps for its backward pass, by ray.  Any
+    thread may take them away: a cube already popped by its backward pass stays alive
+    there, and the memory of one dropped goes back to the stream it came from."""
+
+    def __init__(self):
+        self.by_ray = {}
+        with _lock:
+            _live[next(_order)] = self
+
+    def add(self, r, like):
+        """Ray r's cube, None where there is no room for it."""
+        try:
+            cube = torch.empty_like(like)
+        except torch.OutOfMemoryError:
+            return None
+        with _lock:
+            self.by_ray[r] = cube
+        return cube
+
+    def pop(self, r):
+        with _lock:
+            return self.by_ray.pop(r, None)
+
+    def held(self, device):
+        return sum(t.numel() * t.element_size() for t in self.by_ray.values() if t.device == device)
+
+
+_lock = threading.RLock()
+_order = itertools.count()
+_live = weakref.WeakValueDictionary()       # every solution's _Cubes, oldest first
+
+
+def _give_back(device, most=0):
+    """Drops cubes, the oldest solution's first, until at most `most` bytes are kept on
+    the device: (the bytes still kept, whether any went)."""
+    with _lock:
+        live = [c for _, c in sorted(_live.items())]
+        held = [c.held(device) for c in live]
+        total, gone = sum(held), False
+        for c, n in zip(live, held):
+            if n and total > most:
+                c.by_ray.clear()
+                total, gone = total - n, True
+    return total, gone
+
+
+def _alloc(device, make):
+    """make(), once more without the kept cubes if it finds no memory."""
+    try:
+        return make()
+    except torch.OutOfMemoryError:
+        if not _give_back(device)[1]:
+            raise
+    return make()
+
+
 def _kept_cubes(chi, nray):
-    """How many of nray rays keep their intensity cube: a quarter of the device memory free
-    now (the driver's and the caching allocator's)."""
-    free = torch.cuda.mem_get_info(chi.device)[0]
-    free += torch.cuda.memory_reserved(chi.device) - torch.cuda.memory_allocated(chi.device)
-    return min(nray, free // 4 // max(1, chi.numel() * chi.element_size()))
+    """How many of nray rays keep their intensity cube: all solutions' cubes together at
+    most half of the memory (the driver's free and the caching allocator's) that
+    would be left with no cube kept, after what the backward pass takes (the cotangents
+    of chi and S, a patch and planes: three cubes) and as much again as this process
+    holds otherwise, for the backward pass of the caller's own graph.  Earlier solutions
+    give theirs back where that has become less than they keep, so that a graph of many
+    solutions ends with the memory that the checkpoints alone take."""
+    cube = max(1, chi.numel() * chi.element_size())
+    held = _give_back(chi.device, most=1 << 62)[0]
+    used = torch.cuda.memory_allocated(chi.device) - held
+    free = torch.cuda.mem_get_info(chi.device)[0] + torch.cuda.memory_reserved(chi.device) - used
+    most = max(0, (free - 3 * cube - used) // 2)
+    held = _give_back(chi.device, most)[0]
+    return max(0, min(nray, (most - held) // cube))
 
 
 class _FormalSolution(torch.autograd.Function):
@@ -152,16 +231,21 @@ class _FormalSolution(torch.autograd.Function):
     def forward(fctx, rs, want_J, rays, grad, chi, S, gc_up, gs_up, gi_up, gc_dn, gs_dn, gi_dn):
         ghosts = ((gc_up, gs_up, gi_up), (gc_dn, gs_dn, gi_dn))
         nz, nf, ny, nx = chi.shape
-        exits = torch.zeros((len(rs.vec), nf, ny, nx), dtype=chi.dtype, device=chi.device)
-        J = torch.zeros_like(chi) if want_J else None
+        new = lambda shape: _alloc(chi.device, lambda: torch.empty(shape, dtype=chi.dtype, device=chi.device))
+        exits = new((len(rs.vec), nf, ny, nx)).zero_()
+        J = new(chi.shape).zero_() if want_J else None
         npatch = (nz + rs.patch - 1) // rs.patch
-        ckpt, cubes = {}, {}
-        keep = _kept_cubes(chi, len(rays)) if grad and not want_J else 0
+        ckpt = {r: new((max(npatch - 1, 1), nf, ny, nx)) for r in rays}
+        cubes, keep = None, 0
+        if grad and not want_J:
+            keep = _kept_cubes(chi, len(rays)) if rs.keep == "auto" else min(rs.keep, len(rays))
+            cubes = _Cubes()
         for r in rays:
-            ckpt[r] = torch.empty((max(npatch - 1, 1), nf, ny, nx), dtype=chi.dtype, device=chi.device)
-            if len(cubes) < keep and r not in cubes:
-                cubes[r] = torch.empty_like(chi)
-            rs.sweep_checkpointed(r, chi, S, ghosts, ckpt[r], exits[r], J=J, cube=cubes.get(r))
+            cube = None
+            if keep > 0:
+                cube = cubes.add(r, chi)
+                keep = keep - 1 if cube is not None else 0
+            rs.sweep_checkpointed(r, chi, S, ghosts, ckpt[r], exits[r], J=J, cube=cube)
         fctx.rs, fctx.rays, fctx.ckpt, fctx.cubes = rs, rays, ckpt, cubes
         fctx.save_for_backward(chi, S, gc_up, gs_up, gi_up, gc_dn, gs_dn, gi_dn)
         if want_J:
@@ -179,8 +263,9 @@ class _FormalSolution(torch.autograd.Function):
             J_bar = None
         if J_bar is not None:
             J_bar = J_bar.contiguous()
-        chibar, Sbar = torch.zeros_like(chi), torch.zeros_like(S)
-        gbars = tuple(tuple(torch.zeros_like(t) for t in g) for g in ghosts)
+        zeros = lambda like: _alloc(chi.device, lambda: torch.zeros_like(like))
+        chibar, Sbar = zeros(chi), zeros(S)
+        gbars = tuple(tuple(zeros(t) for t in g) for g in ghosts)
         if exit_bar is not None:
             exit_bar = exit_bar.contiguous()
             live = (exit_bar.flatten(1).abs().amax(dim=1) > 0).cpu().numpy()
@@ -188,15 +273,16 @@ class _FormalSolution(torch.autograd.Function):
             live = np.zeros(len(rs.vec), bool)
         scratch = work = None
         for r in rays:
+            cube = None if cubes is None else cubes.pop(r)      # freed once its ray is done
             if not live[r] and J_bar is None:
                 continue
-            if scratch is None and r not in cubes:
-                scratch = torch.empty((min(rs.patch, chi.shape[0]),) + tuple(chi.shape[1:]), dtype=chi.dtype,
-                                      device=chi.device)
+            if scratch is None and cube is None:
+                shape = (min(rs.patch, chi.shape[0]),) + tuple(chi.shape[1:])
+                scratch = _alloc(chi.device, lambda: torch.empty(shape, dtype=chi.dtype, device=chi.device))
             if work is None:
-                work = tuple(torch.zeros_like(gc_up) for _ in range(3))
+                work = tuple(zeros(gc_up) for _ in range(3))
             rs.adjoint_checkpointed(r, chi, S, ghosts, ckpt[r], scratch, gbars, chibar, Sbar, Jbar=J_bar,
-                                    exit_bar=exit_bar[r] if live[r] else None, work=work, cube=cubes.get(r))
+                                    exit_bar=exit_bar[r] if live[r] else None, work=work, cube=cube)
         fctx.ckpt = fctx.cubes = None
         (gcb_u, gsb_u, gib_u), (gcb_d, gsb_d, gib_d) = gbars
         return None, None, None, None, chibar, Sbar, gcb_u, gsb_u, gib_u, gcb_d, gsb_d, gib_d

@@ -278,7 +278,7 @@ def test_nothing_is_kept_without_a_gradient(ctx, monkeypatch):
     """Under no_grad, and with no input that needs a gradient, no intensity cube is
     written: the exit planes are the same bits as those of a differentiated call."""
     from dispatch_amd import adjoint, synth
-    box = synth.make_box(nx=12, ny=10, nz=9, nf=6, seed=3)
+    box = synth.make_box(nx=24, ny=20, nz=9, nf=6, seed=3)
     chi, S = synth.build_cubes(box, torch.float32)
     gh = synth.ghost_planes(box, chi, torch.float32)
     vecs, wj = synth.gauss_rays(2)
@@ -294,3 +294,49 @@ def test_nothing_is_kept_without_a_gradient(ctx, monkeypatch):
     b = adjoint.formal_solution(rs, chi, S, gh["up"], gh["down"])
     assert asked == [len(vecs)] and not a.requires_grad and not b.requires_grad
     assert torch.equal(a, ref) and torch.equal(b, ref)
+
+
+@pytest.mark.parametrize("case", ["none", "two", "given back", "no room", "waiting"])
+def test_cubes_are_a_shortcut_only(ctx, monkeypatch, case):
+    """RaySet.keep, cubes given back between the passes, an allocation that fails and
+    another solution's cubes waiting: the gradient's bits are those with nothing kept, and
+    nothing stays kept after the backward passes."""
+    from dispatch_amd import adjoint, synth
+    box = synth.make_box(nx=24, ny=20, nz=13, nf=6, seed=5)
+    chi, S = synth.build_cubes(box, torch.float32)
+    gh = synth.ghost_planes(box, chi, torch.float32)
+    vecs, wj = synth.gauss_rays(2)
+    up = [r for r, v in enumerate(vecs) if v[2] > 0]
+    g = torch.Generator(device="cuda").manual_seed(4)
+    cot = torch.rand((len(vecs),) + tuple(chi.shape[1:]), generator=g, device="cuda")
+
+    def solve(keep):
+        rs = adjoint.RaySet(ctx, vecs, wj, box.ds, box.chi500, [synth.chi500_upwind(box, v) for v in vecs],
+                            box.g500_bot, box.g500_top, patch=5, keep=keep)
+        leaves = [t.detach().clone().requires_grad_() for t in (chi, S, *gh["up"])]
+        return leaves, adjoint.formal_solution(rs, *leaves[:2], leaves[2:], gh["down"], rays=up)
+
+    held = lambda: sum(c.held(chi.device) for c in list(adjoint._live.values()))
+    size = chi.numel() * chi.element_size()
+    ref, e = solve(0)
+    assert held() == 0
+    e.backward(cot)
+    if case == "no room":
+        def full(t):
+            raise torch.OutOfMemoryError("no room")
+        monkeypatch.setattr(adjoint.torch, "empty_like", full)
+    one, e1 = solve({"none": 0, "two": 2}.get(case, "auto"))
+    want = {"none": 0, "two": 2, "no room": 0}.get(case, len(up)) * size
+    assert held() == want
+    sets = [(one, e1)]
+    if case == "waiting":
+        sets.append(solve("auto"))
+        assert held() == 2 * want
+    if case == "given back":
+        adjoint._give_back(chi.device)
+        assert held() == 0
+    for leaves, ex in sets:
+        ex.backward(cot)
+        for a, b in zip(ref, leaves):
+            assert torch.equal(a.grad, b.grad)
+    assert held() == 0
