@@ -443,6 +443,8 @@ int m3drt_bb_opacity(m3drt_ctx *ctx, const m3drt_bb_opacity_args *r) {
   if ((r->flags & M3DRT_BBOP_SPLIT) && (!r->split_opac1 || !r->split_opac2 || !r->split_chi1 ||
                                         !r->split_chi2 || !r->split_id || !r->split_chi_id))
     return set_error(M3DRT_EINVAL, "m3drt_bb_opacity: split tracking needs its six arrays");
+  if (r->flags & M3DRT_BBOP_TRACK)
+    return set_error(M3DRT_EINVAL, "m3drt_bb_opacity: M3DRT_BBOP_TRACK is m3drt_window_opacity's");
   if (r->wphi_line && (!r->wphi || !r->wq))
     return set_error(M3DRT_EINVAL, "m3drt_bb_opacity: wphi needs wphi and wq");
   if (r->sf < 1 || r->sc < 1) return set_error(M3DRT_EINVAL, "m3drt_bb_opacity: strides must be >= 1");
@@ -464,6 +466,9 @@ int m3drt_window_opacity(m3drt_ctx *ctx, const m3drt_bb_opacity_args *r, const m
   if ((r->flags & M3DRT_BBOP_SPLIT) && (!r->split_opac1 || !r->split_opac2 || !r->split_chi1 ||
                                         !r->split_chi2 || !r->split_id || !r->split_chi_id))
     return set_error(M3DRT_EINVAL, "m3drt_window_opacity: split tracking needs its six arrays");
+  if ((r->flags & M3DRT_BBOP_SPLIT) && (r->flags & M3DRT_BBOP_TRACK))
+    return set_error(M3DRT_EINVAL, "m3drt_window_opacity: M3DRT_BBOP_SPLIT writes the tracking arrays, "
+                                   "M3DRT_BBOP_TRACK does not: one of the two");
   if (r->wphi_line) return set_error(M3DRT_EINVAL, "m3drt_window_opacity: no wphi sums (use m3drt_bb_opacity)");
   if (w->flags & ~M3DRT_UNITS_SUPPRESS_MASERS)
     return set_error(M3DRT_EINVAL, "m3drt_window_opacity: flags other than M3DRT_UNITS_SUPPRESS_MASERS");

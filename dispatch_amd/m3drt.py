@@ -673,7 +673,7 @@ def _window_opacity(self, d, chi_cont, Bnu, beta, xhat, ehat, split=None, split_
     the continuum, convert_to_work_units, the split tracking seeded with the continuum,
     the lines with add_largest, and work_to_transfer_units.  xhat receives chi and
     ehat S; split (the six tracking arrays) is overwritten.  track: the same chi and S
-    without writing tracking arrays (bb_rates_window forms them again)."""
+    without writing tracking arrays (bb_rates_window forms them again); not with split."""
     L = _ali_lib()
     if not getattr(L, "_win_ok", False):
         L.m3drt_window_opacity.argtypes = [C.c_void_p, C.POINTER(BbOpacityArgs), C.POINTER(WindowArgs)]

@@ -379,14 +379,17 @@ int m3drt_bb_rates(m3drt_ctx *ctx, const m3drt_bb_rates_args *args);
  * came from m3drt_window_opacity with the same lines, cells and chi_cont (f, cell), Bnu
  * and beta: the tracked contributions are formed again from those, the same values
  * that M3DRT_BBOP_SPLIT would have written, and the six split_ arrays are not used
- * (NULL).  Line scattering and psi flags as there. */
+ * (NULL).  Line scattering and psi flags as there.  They are formed with b: b must be what
+ * it was for the opacities, and a window made with M3DRT_BBOP_LTE (b = 1) is not one
+ * for this call. */
 int m3drt_bb_rates_window(m3drt_ctx *ctx, const m3drt_bb_rates_args *args, const float *chi_cont);
 
 /* ------------------------------------------------------------------ line opacity of a model atom */
 
 #define M3DRT_BBOP_LTE 1    /* b = 1 (the LTE companion set) */
 #define M3DRT_BBOP_SPLIT 2  /* track the largest contribution per point (add_largest) */
-#define M3DRT_BBOP_TRACK 4  /* m3drt_window_opacity: as SPLIT, but the tracking arrays are not written */
+#define M3DRT_BBOP_TRACK 4  /* m3drt_window_opacity alone, not with SPLIT: the same chi and S, the tracking
+                               arrays not written (m3drt_bb_rates_window forms them again) */
 
 typedef struct {
   int32_t nline, nf, ncell, nk, flags, split_offset;

@@ -169,6 +169,34 @@ def test_rates_with_the_tracking_formed_again(ctx, kw, overlap, off):
         assert torch.equal(a, b), (what, float((a - b).abs().max()))
 
 
+def test_tracking_flags_that_contradict_are_refused(ctx):
+    """Tracking arrays together with M3DRT_BBOP_TRACK would stay unwritten, and
+    m3drt_bb_opacity has no such form: both are errors, and nothing is written."""
+    import ctypes as C
+    from dispatch_amd import m3drt, synth
+    from dispatch_amd.ali import NlteProblem
+    p = NlteProblem(ctx, small())
+    w = p.windows[0]
+    l0, l1, nf, nc = w.lines[0], w.lines[-1] + 1, w.nf, p.ncell
+    d = dict(w.const, vproj=(p.vz * (p.vec[0][2] / synth.C_LIGHT)).float().contiguous(), b=p.b, nstar=p.nstar,
+             pop_ratio=p.pop_ratio, inv_df=p.inv_df, e_kT=p.e_kT32, adamp=p.adamp[l0:l1])
+    chi, S = torch.full_like(w.chi_c, 3.0), torch.full_like(w.chi_c, 3.0)
+    sp = {k: torch.full_like(w.chi_c, 3.0) for k in ("split_opac1", "split_opac2", "split_chi1", "split_chi2")}
+    sp.update({k: torch.full((nf, nc), 3, dtype=torch.int32, device="cuda") for k in ("split_id", "split_chi_id")})
+    with pytest.raises(m3drt.M3drtError, match="one of the two"):
+        ctx.window_opacity(d, w.chi_c, w.Bnu, w.beta, chi, S, split=sp, track=True)
+    ptr = lambda t: C.c_void_p(t.data_ptr())
+    a = m3drt.BbOpacityArgs(l1 - l0, nf, nc, p.b.shape[0], m3drt.M3DRT_BBOP_TRACK, 0, 0.0, nc, 1,
+                            *[ptr(d[k]) for k in ("iblue", "ired", "lev_i", "lev_j", "Bij", "lower_off", "q")], None,
+                            None, *[ptr(d[k]) for k in ("b", "nstar", "pop_ratio", "inv_df", "vproj", "e_kT", "adamp")],
+                            ptr(chi), ptr(S), *[None] * 7)
+    with pytest.raises(m3drt.M3drtError, match="m3drt_window_opacity's"):
+        m3drt._check(m3drt._ali_lib().m3drt_bb_opacity(ctx._h, C.byref(a)), "m3drt_bb_opacity")
+    torch.cuda.synchronize()
+    for t in (chi, S, *sp.values()):
+        assert bool((t == 3).all())
+
+
 def test_graph_replays_of_the_rate_pass_match_eager(ctx):
     """AliConfig(graph=True): the rate pass captured once and replayed, with the
     statistical-equilibrium update (eager work) between the replays, gives the eager
