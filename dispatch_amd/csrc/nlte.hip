@@ -5,10 +5,10 @@
 // under-relaxation, particle conservation, population floor and the convergence
 // measure.  Also the rate normalisation of normalize_profiles (377-431).
 //
-// Mapping.  Sixteen lanes per cell, four cells a wavefront.  A workgroup of NT cells
-// keeps every cell's nk x nk matrix, right-hand side and b*n* vector in LDS, one cell
-// after another.  A cell's lanes share its elimination as a 4 x 4 grid over the rows and
-// columns left, and otherwise take its levels in turn; they lie in one wavefront, whose
+// Mapping.  Sixteen lanes per cell, four cells a wavefront (many cells of few levels: four
+// lanes, rate_solve).  A workgroup of NT cells keeps every cell's nk x nk matrix,
+// right-hand side and b*n* vector in LDS, one cell after another.  A cell's lanes share its
+// elimination as a 4 x 4 (2 x 2) grid over the rows and columns left, and otherwise take its levels in turn; they lie in one wavefront, whose
 // LDS accesses are in order, so no barrier is needed between the steps.  Every element
 // sees the operations of the sequential algorithm in its order, so the results are
 // those of one lane per cell.  What bounds it is the latency of the dependent steps
@@ -52,17 +52,19 @@ __device__ __forceinline__ bool better(double va, int ca, double vb, int cb) {
   return a > b || (a == b && ca < cb);
 }
 
-constexpr int kSeLanes = 16;       // lanes of a cell
-constexpr int kSeCells = 40;       // cells of a workgroup, at most
+// cells of a workgroup at most, with LANES lanes a cell
+template <int LANES>
+constexpr int se_cells() { return LANES == 16 ? 40 : 64; }
 
 // doubles of a cell in LDS: matrix, right-hand side, b*n*; odd, so that the cells of a
 // wavefront start on different banks
 __host__ __device__ __forceinline__ int se_stride(int nk) { return (nk * nk + 2 * nk) | 1; }
 
-__global__ void __launch_bounds__(kSeLanes * kSeCells) se_update_kernel(const SeArgs a) {
+template <int LANES>
+__global__ void __launch_bounds__(LANES *se_cells<LANES>()) se_update_kernel(const SeArgs a) {
   extern __shared__ double sm[];
   const int nk = a.nk, NT = a.nt;
-  const int t = threadIdx.x / kSeLanes, p = threadIdx.x % kSeLanes;
+  const int t = threadIdx.x / LANES, p = threadIdx.x % LANES;
   const int c = blockIdx.x * NT + t;
   double *W = sm + (size_t)t * se_stride(nk);    // nk*nk
   double *E = W + (size_t)nk * nk;               // nk
@@ -84,10 +86,10 @@ __global__ void __launch_bounds__(kSeLanes * kSeCells) se_update_kernel(const Se
   if (live) {
     const double ekt = a.e_kT[c];
     auto NS = [&](int i) { return a.nstar[(size_t)i * a.ncell + c]; };
-    for (int e = p; e < nk * nk; e += kSeLanes) W[e] = 0.0;
-    for (int i = p; i < nk; i += kSeLanes) Ev(i) = 0.0;
+    for (int e = p; e < nk * nk; e += LANES) W[e] = 0.0;
+    for (int i = p; i < nk; i += LANES) Ev(i) = 0.0;
     sync();
-    // The rates of sixteen transitions at a time, one a lane, then added in their order:
+    // The rates of as many transitions at a time as lanes, one a lane, then added in their order:
     // lane 0 the upward rate to W(j, i), lane 1 the downward one to W(i, j).
     auto add = [&](int i, int j, double up, double down) {
       if (i == j) {
@@ -98,7 +100,7 @@ __global__ void __launch_bounds__(kSeLanes * kSeCells) se_update_kernel(const Se
       }
       sync();
     };
-    for (int k0 = 0; k0 < a.nrad; k0 += kSeLanes) {
+    for (int k0 = 0; k0 < a.nrad; k0 += LANES) {
       const int kr = k0 + p;
       double r_up = 0.0, r_down = 0.0;
       if (kr < a.nrad && a.active[kr]) {
@@ -121,13 +123,13 @@ __global__ void __launch_bounds__(kSeLanes * kSeCells) se_update_kernel(const Se
           r_down = a.gji[(size_t)kr * a.ncell + c];
         }
       }
-      for (int q = 0; q < kSeLanes && k0 + q < a.nrad; ++q) {
+      for (int q = 0; q < LANES && k0 + q < a.nrad; ++q) {
         if (!a.active[k0 + q]) continue;
-        add(a.ti[k0 + q] - 1, a.tj[k0 + q] - 1, __shfl(r_up, q, kSeLanes), __shfl(r_down, q, kSeLanes));
+        add(a.ti[k0 + q] - 1, a.tj[k0 + q] - 1, __shfl(r_up, q, LANES), __shfl(r_down, q, LANES));
       }
     }
     if (a.cswitch > 0 && a.cup) {
-      for (int q0 = 0; q0 < a.npair; q0 += kSeLanes) {
+      for (int q0 = 0; q0 < a.npair; q0 += LANES) {
         const int q = q0 + p;
         double up = 0.0, down = 0.0;
         if (q < a.npair) {
@@ -138,11 +140,11 @@ __global__ void __launch_bounds__(kSeLanes * kSeCells) se_update_kernel(const Se
             down = cu * (NS(i) / NS(j)) * a.cswitch;
           }
         }
-        for (int m = 0; m < kSeLanes && q0 + m < a.npair; ++m)
-          add(a.pi[q0 + m] - 1, a.pj[q0 + m] - 1, __shfl(up, m, kSeLanes), __shfl(down, m, kSeLanes));
+        for (int m = 0; m < LANES && q0 + m < a.npair; ++m)
+          add(a.pi[q0 + m] - 1, a.pj[q0 + m] - 1, __shfl(up, m, LANES), __shfl(down, m, LANES));
       }
     }
-    for (int i = p; i < nk; i += kSeLanes) {
+    for (int i = p; i < nk; i += LANES) {
       double s = 0.0;
       for (int k = 0; k < nk; ++k) s += Wm(k, i);
       Wm(i, i) = -s;
@@ -153,22 +155,24 @@ __global__ void __launch_bounds__(kSeLanes * kSeCells) se_update_kernel(const Se
     for (int i = 0; i < nk; ++i)
       if (Bv(i) > Bv(pos)) pos = i;
     if (p == 0) Ev(pos) = a.totn[c];
-    for (int j = p; j < nk; j += kSeLanes) {
+    for (int j = p; j < nk; j += LANES) {
       const double bj = Bv(j);
       for (int i = 0; i < nk; ++i) Wm(i, j) = i == pos ? bj : Wm(i, j) * bj;
     }
     sync();
 
     // lineq_no_pivot: Doolittle without pivoting, zero upper entries skipped
-    const int pi = p >> 2, pj = p & 3;
+    constexpr int G = LANES == 16 ? 4 : 2;
+    static_assert(G * G == LANES, "a cell's lanes form a square");
+    const int pi = p / G, pj = p % G;
     for (int k = 0; k < nk - 1; ++k) {
       const double akk = Wm(k, k);
-      for (int i = k + 1 + p; i < nk; i += kSeLanes) Wm(i, k) = Wm(i, k) / akk;
+      for (int i = k + 1 + p; i < nk; i += LANES) Wm(i, k) = Wm(i, k) / akk;
       sync();
-      for (int j = k + 1 + pj; j < nk; j += 4) {
+      for (int j = k + 1 + pj; j < nk; j += G) {
         const double akj = Wm(k, j);
         if (akj != 0)
-          for (int i = k + 1 + pi; i < nk; i += 4) Wm(i, j) = Wm(i, j) - Wm(i, k) * akj;
+          for (int i = k + 1 + pi; i < nk; i += G) Wm(i, j) = Wm(i, j) - Wm(i, k) * akj;
       }
       sync();
     }
@@ -176,7 +180,7 @@ __global__ void __launch_bounds__(kSeLanes * kSeCells) se_update_kernel(const Se
     // on every lane alike
     for (int j = 0; j < nk - 1; ++j) {
       const double ej = Ev(j);
-      for (int i = j + 1 + p; i < nk; i += kSeLanes) Ev(i) = Ev(i) - Wm(i, j) * ej;
+      for (int i = j + 1 + p; i < nk; i += LANES) Ev(i) = Ev(i) - Wm(i, j) * ej;
       sync();
     }
     for (int i = nk - 1; i >= 0; --i) {
@@ -193,7 +197,7 @@ __global__ void __launch_bounds__(kSeLanes * kSeCells) se_update_kernel(const Se
       if (p == 0) atomicMin(a.status, c + 1);
     } else {
       const double eup = a.max_update > 1.0 ? a.max_update : 1.0, elo = 1.0 / eup;
-      for (int i = p; i < nk; i += kSeLanes) {
+      for (int i = p; i < nk; i += LANES) {
         double e = Ev(i);
         if (e < elo || e > eup) clamps++;
         if (e < elo)
@@ -210,7 +214,7 @@ __global__ void __launch_bounds__(kSeLanes * kSeCells) se_update_kernel(const Se
       for (int i = 0; i < nk; ++i) sum += Ev(i) * NS(i);
       const double norm = a.totn[c] / sum;
       sync();
-      for (int i = p; i < nk; i += kSeLanes) {
+      for (int i = p; i < nk; i += LANES) {
         const size_t o = (size_t)i * a.ncell + c;
         double bn = Ev(i) * norm;
         if (a.nstar[o] > 0) bn = fmax(bn, fmin(1.0, a.min_pop_frac * a.totn[c] / a.nstar[o]));
@@ -336,7 +340,14 @@ __global__ void __launch_bounds__(256) normalize_kernel(int nrad, int nline, int
 int rate_solve(m3drt_ctx *ctx, const m3drt_rate_solve_args *r, m3drt_rate_solve_result *res) {
   const int nk = r->nk;
   const size_t per_cell = ((size_t)nk * nk + 2 * (size_t)nk + 2) * sizeof(double) + 2 * sizeof(int);
-  int nt = (int)std::min<size_t>(kSeCells, (size_t)ctx->lds_max / per_cell);
+  // Few levels leave most of sixteen lanes idle, and more cells than the chip holds at
+  // sixteen lanes then wait: four lanes.  Measured (4 lanes against 16, us): 432 000 cells
+  // of 3 levels 214 / 592, 6 levels 322 / 928, 11 levels 1133 / 1829, 16 levels
+  // 3442 / 3818, 21 levels 7780 / 5397; 30 000 cells of 3 levels 112 / 128, 9 levels
+  // 141 / 181, 16 levels 326 / 348; 10 000 cells of 6 levels 124 / 111, 9 levels 133 / 120,
+  // 16 levels 211 / 175.  (One lane: 171 us for 432 000 cells of 3 levels, 373 for 6.)
+  const int lanes = nk <= 16 && r->ncell > 16384 ? 4 : 16;
+  int nt = (int)std::min<size_t>(lanes == 4 ? se_cells<4>() : se_cells<16>(), (size_t)ctx->lds_max / per_cell);
   if (nt >= 4) nt -= nt % 4;
   if (nt < 1) return set_error(M3DRT_ELIMIT, "m3drt_rate_solve_f64: nk too large for the LDS");
   const int nblk = (r->ncell + nt - 1) / nt;
@@ -372,9 +383,13 @@ int rate_solve(m3drt_ctx *ctx, const m3drt_rate_solve_args *r, m3drt_rate_solve_
   a.tmax_update = r->tmax_update;
   a.blk_err = blk_err; a.blk_cell = blk_cell; a.blk_lvl = blk_lvl; a.blk_lerr = blk_lerr;
   a.blk_lcell = blk_lcell; a.nclamp = nclamp; a.status = status;
-  M3DRT_HIP(hipFuncSetAttribute((const void *)se_update_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)lds));
-  hipLaunchKernelGGL(se_update_kernel, dim3(nblk), dim3(nt * kSeLanes), lds, ctx->stream, a);
+  auto run = [&](auto kern) -> int {
+    M3DRT_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(kern, dim3(nblk), dim3(nt * lanes), lds, ctx->stream, a);
+    return M3DRT_OK;
+  };
+  rc = lanes == 4 ? run(se_update_kernel<4>) : run(se_update_kernel<16>);
+  if (rc) return rc;
   M3DRT_HIP(hipGetLastError());
   hipLaunchKernelGGL(se_final_kernel, dim3(nk + 1), dim3(256), 0, ctx->stream, nblk, nk, blk_err, blk_cell, blk_lvl,
                      blk_lerr, blk_lcell, out, iout);

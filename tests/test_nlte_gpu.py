@@ -89,3 +89,33 @@ def test_rate_solve_sizes(ctx, monkeypatch, nbound, nline, ncont, ncell):
     assert (r["epos"], r["elvl"]) == (rref["epos"], rref["elvl"])
     assert r["nclamp"] == rref["nclamp"]
     assert np.allclose(r["lvlerr"], rref["lvlerr"], rtol=1e-8, atol=1e-10)
+
+
+@pytest.mark.parametrize("nbound,nline,ncont,ncell", [(2, 1, 2, 16385), (4, 5, 4, 16500), (8, 14, 8, 20000), (15, 60, 15, 16390),
+                                                      (16, 60, 16, 16390)])
+def test_rate_solve_of_many_cells_equals_few_at_a_time(ctx, monkeypatch, nbound, nline, ncont, ncell):
+    """Four lanes a cell take many cells of up to 16 levels, sixteen the others, with the
+    same operations in the same order: one call over all cells against calls of at most
+    16 384, the populations bit for bit and the largest changes and their cells."""
+    import functools
+    from dispatch_amd import m3drt, synth
+    monkeypatch.setattr(synth, "make_atom", functools.partial(synth.make_atom, nbound=nbound))
+    c = make_se_case(ncell=ncell, seed=nbound, nline=nline, ncont=ncont)
+    print(f"rate solve of many cells nbound={nbound} ncell={ncell}", flush=True)
+    atom = m3drt.AtomOnDevice(c["atom"])
+
+    def solve(cells):
+        d = lambda k, dt: dev(c[k][..., cells], dt)
+        b = d("b", torch.float64)
+        r = ctx.rate_solve(atom, d("e_kT", torch.float64), d("T", torch.float64), d("totn", torch.float64),
+                           d("nstar", torch.float64), b, d("gij", torch.float32), d("gji", torch.float32),
+                           d("cup", torch.float64))
+        return b, r
+
+    b, r = solve(slice(0, ncell))
+    parts = [(c0, *solve(slice(c0, min(ncell, c0 + 8192)))) for c0 in range(0, ncell, 8192)]
+    assert torch.equal(b, torch.cat([p[1] for p in parts], 1))
+    assert r["nclamp"] == sum(p[2]["nclamp"] for p in parts)
+    c0, _, best = max(parts, key=lambda p: abs(p[2]["maxerr"]))
+    assert (r["maxerr"], r["epos"], r["elvl"]) == (best["maxerr"], best["epos"] + c0, best["elvl"])
+    assert np.max(np.abs(r["lvlerr"])) == np.max(np.abs([p[2]["lvlerr"] for p in parts]))
