@@ -3,6 +3,7 @@
 // reference's HOP C ABI (HOP/standalone/hop_c_api.f90:1-18): int status, message
 // by m3drt_last_error, no process exit in library code.
 #include "m3drt_internal.hpp"
+#include <algorithm>
 #include <cstring>
 #include <cstdio>
 #include <string>
@@ -19,6 +20,38 @@ int set_error(int code, const std::string &msg) {
 int hip_check(hipError_t e, const char *what) {
   std::string m = std::string(what) + ": " + hipGetErrorString(e);
   return set_error(e == hipErrorOutOfMemory ? M3DRT_ENOMEM : M3DRT_EDEVICE, m);
+}
+
+static size_t scratch_rounded(size_t bytes) { return (bytes + (1u << 20) - 1) & ~(size_t)((1u << 20) - 1); }
+
+size_t offer_scratch(m3drt_ctx *ctx, size_t least, size_t want) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(ctx->stream, &cs) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  const bool capturing = cs != hipStreamCaptureStatusNone;
+  if (want > ctx->scratch_bytes && want < ctx->scratch_refused && !ctx->scratch_fixed && !capturing) {
+    void *p = nullptr;
+    const size_t rounded = scratch_rounded(want);
+    if (hipMalloc(&p, rounded) != hipSuccess) {
+      (void)hipGetLastError();
+      ctx->scratch_refused = want;
+    } else {
+      if (ctx->scratch_captured) {
+        ctx->retired.push_back(ctx->scratch);  // as in ensure_scratch
+      } else if (ctx->scratch) {
+        (void)hipStreamSynchronize(ctx->stream);
+        (void)hipFree(ctx->scratch);
+      }
+      ctx->scratch = p;
+      ctx->scratch_bytes = rounded;
+      ctx->scratch_captured = false;
+    }
+  }
+  if (ctx->scratch_bytes < least) return 0;
+  if (capturing && !ctx->scratch_fixed) ctx->scratch_captured = true;
+  return std::min(want, ctx->scratch_bytes);
 }
 
 int ensure_scratch(m3drt_ctx *ctx, size_t bytes) {
@@ -46,7 +79,7 @@ int ensure_scratch(m3drt_ctx *ctx, size_t bytes) {
     ctx->scratch_bytes = 0;
     ctx->scratch_captured = false;
   }
-  const size_t rounded = (bytes + (1u << 20) - 1) & ~(size_t)((1u << 20) - 1);
+  const size_t rounded = scratch_rounded(bytes);
   M3DRT_HIP(hipMalloc(&ctx->scratch, rounded));
   ctx->scratch_bytes = rounded;
   return M3DRT_OK;

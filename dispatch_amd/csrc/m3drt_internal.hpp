@@ -13,6 +13,7 @@ struct m3drt_ctx {
   void *scratch = nullptr;   // per-call scratch (dt500, rc per cell, ...); grown on demand
   size_t scratch_bytes = 0;
   bool scratch_captured = false;  // a stream capture recorded launches that use `scratch`
+  size_t scratch_refused = ~(size_t)0;  // the smallest size offer_scratch could not grow to
   bool scratch_fixed = false;     // `scratch` is a caller-fixed buffer for this call: never grown
   std::vector<void *> retired;    // outgrown scratch buffers captured graphs may still use
   int lds_max = 0;           // dynamic LDS bytes available per workgroup
@@ -30,6 +31,10 @@ int hip_check(hipError_t e, const char *what);
 // capture is refused.  With a fixed buffer (m3drt_sc_sweep_noalloc) a larger need
 // is refused with M3DRT_ELIMIT.
 int ensure_scratch(m3drt_ctx *ctx, size_t bytes);
+// For callers that work with less: as much of `want` bytes as ctx->scratch holds after
+// growing where that is allowed and succeeds (the buffer at hand stays where it does not,
+// and a size refused once is not tried again); 0 if that is less than `least`.  Sets no error.
+size_t offer_scratch(m3drt_ctx *ctx, size_t least, size_t want);
 // the sweep entry point's checks and dispatch (m3drt_sc_sweep, m3drt_sc_sweep_noalloc)
 int sc_sweep_checked(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const m3drt_sweep_bufs *b, const char *who);
 // the fixed device scratch of m3drt_sc_sweep_noalloc: its address on `device`

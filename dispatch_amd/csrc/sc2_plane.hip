@@ -162,8 +162,8 @@ int sweep_sc2_plane(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const m3drt_sweep
   const uint64_t gspan = (uint64_t)(nx - 1) * d->gs_x + (uint64_t)(ny - 1) * d->gs_y + nf;
   if (span >= (1ull << 31) || gspan >= (1ull << 31) || (uint64_t)nxy * nf >= (1ull << 31)) return -1;
 
-  // An exit plane written over the ghost plane: safe while other launches lie between
-  // the reads and the writes, so not with a single plane.
+  // An exit plane written over the ghost plane: safe while other launches lie between a
+  // frequency's reads and its writes, so not with a single plane.
   if (nz == 1 && b->exit_I) {
     const char *e = static_cast<const char *>(b->exit_I);
     for (const void *p : {b->ghost_chi, b->ghost_S, b->ghost_I}) {
@@ -172,11 +172,22 @@ int sweep_sc2_plane(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const m3drt_sweep
     }
   }
 
-  const size_t nprep = (size_t)nxy * (nz + 1), nI = (size_t)nxy * nf;
-  if (ensure_scratch(ctx, sizeof(T) * (2 * nprep + 2 * nI))) {
-    (void)hipGetLastError();  // no room (a fixed or captured scratch, no memory): the other kernels need less
-    return -1;
+  // The frequencies in runs whose two intensity planes the scratch holds: all of them
+  // where it may grow (to 512 MiB of planes), the ones that fit beside the preparation
+  // where it may not (m3drt_sc_sweep_noalloc's 32 MiB, a capture, no memory).  They are
+  // independent, so the runs change no value: 1024 frequencies of the 120 x 120 x 23 slab
+  // take four runs of 256 in the 32 MiB.
+  const size_t nprep = (size_t)nxy * (nz + 1), prep = 2 * nprep * sizeof(T), per_f = 2 * (size_t)nxy * sizeof(T);
+  const size_t most = std::min<size_t>(nf, std::max<size_t>(64, ((size_t)512 << 20) / per_f / 64 * 64));
+  const size_t room = offer_scratch(ctx, prep + 16 * per_f, prep + most * per_f);
+  if (!room) return -1;
+  int run = (int)((room - prep) / per_f);
+  if (run < nf) {
+    run -= run % (run >= 64 ? 64 : 16);
+    const int nrun = (nf + run - 1) / run;
+    run = std::min(run, ((nf + nrun - 1) / nrun + 15) / 16 * 16);
   }
+  const size_t nI = (size_t)nxy * run;
   T *dt500 = static_cast<T *>(ctx->scratch), *rc = dt500 + nprep, *I0 = rc + nprep, *I1 = I0 + nI;
   const Sc2Geom g = sc2_geometry(d);
   const int st = sc2_prep<T>(ctx, d, b->chi500, b->chi500_up, b->g500, dt500, rc);
@@ -188,7 +199,7 @@ int sweep_sc2_plane(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const m3drt_sweep
   T *const Iout = static_cast<T *>(b->I_out), *const Psiout = rates ? static_cast<T *>(b->Psi_out) : nullptr;
   a.split = (d->flags & M3DRT_SPLIT_RATES) ? 1 : 0;
   const bool plain = J && !PsiJ && !Iout && !Psiout && !a.split;
-  a.nf = nf; a.nx = nx; a.ny = ny; a.xo = g.xo; a.yo = g.yo;
+  a.nx = nx; a.ny = ny; a.xo = g.xo; a.yo = g.yo;
   a.cs_x = (uint32_t)d->cs_x; a.cs_y = (uint32_t)d->cs_y;
   a.gs_x = (uint32_t)d->gs_x; a.gs_y = (uint32_t)d->gs_y;
   // the stencil in FP32 as the reference casts it (FP64 sweep: in FP64)
@@ -202,13 +213,6 @@ int sweep_sc2_plane(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const m3drt_sweep
   a.imax = f64 ? (T)d->maser_Inu_max : (T)(float)d->maser_Inu_max;
   a.wj = (T)d->wj;
 
-  // frequencies a wave takes: the widest of 64, 32, 16 that leaves no more lanes idle
-  int fw = 64;
-  auto lanes = [&](int w) { return (nf + w - 1) / w * w; };
-  for (int w : {32, 16})
-    if (lanes(w) * 9 <= lanes(fw) * 8) fw = w;
-  a.nfc = (nf + fw - 1) / fw;
-  a.nxb = (nx + 256 / fw - 1) / (256 / fw);
   // Rows a lane takes: one where the plane barely fills the chip (a lane's rows follow
   // one another, each a round trip to the cache), up to eight where the points keep
   // the memory busy and the three rows a strip re-reads count.  Measured (FP32, 20 to
@@ -218,45 +222,55 @@ int sweep_sc2_plane(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const m3drt_sweep
   const int64_t pb = nxy * nf * (int64_t)sizeof(T) >> 20;
   int L = lenv ? atoi(lenv) : pb >= 12 ? 8 : pb >= 4 ? 4 : pb >= 1 ? 2 : 1;
   L = L >= 8 ? 8 : L >= 4 ? 4 : L >= 2 ? 2 : 1;
-  a.total = a.nxb * ((ny + L - 1) / L) * a.nfc;
-  a.per = (a.total + kXcds - 1) / kXcds;
-  if (getenv("M3DRT_VERBOSE"))
-    fprintf(stderr, "[m3drt] sc2 plane %s nf=%d plane=%dx%d nz=%d: %d workgroups a plane, %d frequencies a wave, strip %d\n",
-            f64 ? "f64" : "f32", nf, nx, ny, nz, a.total, fw, L);
   const int dir = d->dir > 0 ? 1 : -1;
-  for (int step = 0; step < nz; ++step) {
-    const int z = dir > 0 ? step : nz - 1 - step;
-    const int64_t zo = (int64_t)z * d->cs_z, uo = (int64_t)(z - dir) * d->cs_z;
-    auto at = [&](T *p) { return p ? p + zo : nullptr; };
-    a.chi = static_cast<const T *>(b->chi) + zo;
-    a.S = static_cast<const T *>(b->S) + zo;
-    a.dt500 = dt500 + (int64_t)z * nxy;
-    a.rc = rc + (int64_t)z * nxy;
-    if (step == 0) {
-      a.uchi = static_cast<const T *>(b->ghost_chi);
-      a.uS = static_cast<const T *>(b->ghost_S);
-      a.uI = static_cast<const T *>(b->ghost_I);
-      a.urc = rc + (int64_t)nz * nxy;
-      a.us_x = a.is_x = a.gs_x;
-      a.us_y = a.is_y = a.gs_y;
-    } else {
-      a.uchi = static_cast<const T *>(b->chi) + uo;
-      a.uS = static_cast<const T *>(b->S) + uo;
-      a.uI = step & 1 ? I0 : I1;
-      a.urc = rc + (int64_t)(z - dir) * nxy;
-      a.us_x = a.cs_x; a.us_y = a.cs_y;
-      a.is_x = (uint32_t)nf; a.is_y = (uint32_t)nf * nx;
+  for (int f0 = 0; f0 < nf; f0 += run) {
+    a.nf = std::min(run, nf - f0);
+    // frequencies a wave takes: the widest of 64, 32, 16 that leaves no more lanes idle
+    int fw = 64;
+    auto lanes = [&](int w) { return (a.nf + w - 1) / w * w; };
+    for (int w : {32, 16})
+      if (lanes(w) * 9 <= lanes(fw) * 8) fw = w;
+    a.nfc = (a.nf + fw - 1) / fw;
+    a.nxb = (nx + 256 / fw - 1) / (256 / fw);
+    a.total = a.nxb * ((ny + L - 1) / L) * a.nfc;
+    a.per = (a.total + kXcds - 1) / kXcds;
+    if (getenv("M3DRT_VERBOSE"))
+      fprintf(stderr, "[m3drt] sc2 plane %s nf=%d+%d of %d plane=%dx%d nz=%d: %d workgroups a plane, %d frequencies a wave, strip %d\n",
+              f64 ? "f64" : "f32", f0, a.nf, nf, nx, ny, nz, a.total, fw, L);
+    for (int step = 0; step < nz; ++step) {
+      const int z = dir > 0 ? step : nz - 1 - step;
+      const int64_t zo = (int64_t)z * d->cs_z + f0, uo = (int64_t)(z - dir) * d->cs_z + f0;
+      auto at = [&](void *p) { return p ? static_cast<T *>(p) + zo : nullptr; };
+      a.chi = static_cast<const T *>(b->chi) + zo;
+      a.S = static_cast<const T *>(b->S) + zo;
+      a.dt500 = dt500 + (int64_t)z * nxy;
+      a.rc = rc + (int64_t)z * nxy;
+      if (step == 0) {
+        a.uchi = static_cast<const T *>(b->ghost_chi) + f0;
+        a.uS = static_cast<const T *>(b->ghost_S) + f0;
+        a.uI = static_cast<const T *>(b->ghost_I) + f0;
+        a.urc = rc + (int64_t)nz * nxy;
+        a.us_x = a.is_x = a.gs_x;
+        a.us_y = a.is_y = a.gs_y;
+      } else {
+        a.uchi = static_cast<const T *>(b->chi) + uo;
+        a.uS = static_cast<const T *>(b->S) + uo;
+        a.uI = step & 1 ? I0 : I1;
+        a.urc = rc + (int64_t)(z - dir) * nxy;
+        a.us_x = a.cs_x; a.us_y = a.cs_y;
+        a.is_x = (uint32_t)a.nf; a.is_y = (uint32_t)a.nf * nx;
+      }
+      a.nI = step & 1 ? I1 : I0;
+      a.J = at(J); a.PsiJ = at(PsiJ); a.Iout = at(Iout); a.Psiout = at(Psiout);
+      a.Irem = a.split ? at(b->Irem_out) : nullptr;
+      a.esc = a.split ? at(b->escape_out) : nullptr;
+      a.exitI = step == nz - 1 && b->exit_I ? static_cast<T *>(b->exit_I) + f0 : nullptr;
+      if (L == 8) launch_plane<T, 8>(ctx->stream, a, a.per * kXcds, fw, plain);
+      else if (L == 4) launch_plane<T, 4>(ctx->stream, a, a.per * kXcds, fw, plain);
+      else if (L == 2) launch_plane<T, 2>(ctx->stream, a, a.per * kXcds, fw, plain);
+      else launch_plane<T, 1>(ctx->stream, a, a.per * kXcds, fw, plain);
+      M3DRT_HIP(hipGetLastError());
     }
-    a.nI = step & 1 ? I1 : I0;
-    a.J = at(J); a.PsiJ = at(PsiJ); a.Iout = at(Iout); a.Psiout = at(Psiout);
-    a.Irem = a.split ? at(static_cast<T *>(b->Irem_out)) : nullptr;
-    a.esc = a.split ? at(static_cast<T *>(b->escape_out)) : nullptr;
-    a.exitI = step == nz - 1 ? static_cast<T *>(b->exit_I) : nullptr;
-    if (L == 8) launch_plane<T, 8>(ctx->stream, a, a.per * kXcds, fw, plain);
-    else if (L == 4) launch_plane<T, 4>(ctx->stream, a, a.per * kXcds, fw, plain);
-    else if (L == 2) launch_plane<T, 2>(ctx->stream, a, a.per * kXcds, fw, plain);
-    else launch_plane<T, 1>(ctx->stream, a, a.per * kXcds, fw, plain);
-    M3DRT_HIP(hipGetLastError());
   }
   return M3DRT_OK;
 }

@@ -110,3 +110,84 @@ def test_noalloc_refuses_beyond_its_fixed_size(ctx):
                  ds=box.ds, vec=v, wj=1.0, J=J)
     torch.cuda.synchronize()
     assert float(J.abs().max()) > 0.0
+
+
+def _slab(nx, ny, nz, nf, dtype, seed=1):
+    """A slab in the reference layout (nz, ny, nx, nf) and its directions' geometry."""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    r = lambda *s: (torch.rand(s, generator=g, device="cuda") + 0.5)
+    cube = lambda k: (r(nz, ny, nx, nf) * k).to(dtype)
+    plane = lambda k: (r(ny, nx, nf) * k).to(dtype)
+    args = (cube(1e-7), cube(1.0), plane(1e-7), plane(1.0), plane(1.0), r(nz, ny, nx) * 1e-7, r(nz, ny, nx) * 1e-7,
+            r(ny, nx) * 1e-7)
+    return args, dict(dir=1, ds=(50e5, 50e5, 10e5), vec=(0.3, -0.4, 0.866), layout="reference", wj=0.25)
+
+
+@pytest.mark.parametrize("nf,nx,ny,nz,dtype", [(250, 120, 120, 3, torch.float32), (300, 120, 120, 3, torch.float32),
+                                               (1024, 120, 120, 2, torch.float32), (170, 120, 120, 3, torch.float64),
+                                               (40, 120, 120, 230, torch.float32), (97, 101, 67, 250, torch.float32)])
+def test_frequencies_in_runs_have_the_same_bits(ctx, nf, nx, ny, nz, dtype):
+    """Slabs with the frequencies at unit stride whose two intensity planes fit the fixed
+    array, in two to eight runs of frequencies, with run lengths that do not divide nf:
+    the allocating sweep's bits, and no error left behind by a call that succeeds."""
+    args, geo = _slab(nx, ny, nz, nf, dtype)
+    with pytest.raises(m3drt.M3drtError):
+        ctx.sc_sweep(*args, **dict(geo, dir=0), exit_I=torch.zeros_like(args[4]))
+    left = m3drt.last_error()
+    out = []
+    for noalloc in (False, True):
+        J, ex = torch.full_like(args[0], 0.125), torch.zeros_like(args[4])
+        ctx.sc_sweep(*args, J=J, exit_I=ex, noalloc=noalloc, **geo)
+        torch.cuda.synchronize()
+        assert m3drt.last_error() == left
+        out.append((J, ex))
+    assert float(out[0][1].abs().max()) > 0
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
+
+
+def test_capture_with_little_scratch_has_the_same_bits():
+    """A fresh context whose scratch holds the planes of a few frequencies only, captured:
+    the capture takes them in runs, and its replays give the eager call's bits."""
+    args, geo = _slab(60, 60, 5, 200, torch.float32)
+    ctx = m3drt.Context(0)
+    try:
+        few = [t[..., :16].contiguous() for t in args[:5]]
+        ctx.sc_sweep(*few, *args[5:], J=torch.zeros_like(few[0]), **geo)      # 1 MiB of scratch
+        J = torch.zeros_like(args[0])
+        s, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(s):
+            with torch.cuda.graph(g, stream=s):
+                J.zero_()
+                ctx.sc_sweep(*args, J=J, **geo)
+        torch.cuda.synchronize()
+        ref = torch.zeros_like(J)
+        ctx.sc_sweep(*args, J=ref, **geo)                                     # the scratch grows
+        torch.cuda.synchronize()
+        assert float(ref.abs().max()) > 0
+        for rep in range(3):
+            J.fill_(float("nan"))
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(J, ref), rep
+            ctx.sc_sweep(*args, J=torch.zeros_like(J), **geo)
+            torch.cuda.synchronize()
+    finally:
+        ctx.close()
+
+
+@pytest.mark.parametrize("nz", [1, 2])
+@pytest.mark.parametrize("noalloc", [False, True])
+def test_exit_plane_over_the_ghost_plane(ctx, nz, noalloc):
+    """exit_I laid over ghost_I, as a column of slabs hands its planes on: the values of a
+    call with a plane of its own, with one plane (where other workgroups could read what
+    has been written) and with more."""
+    args, geo = _slab(48, 40, nz, 64, torch.float32)
+    ex = torch.zeros_like(args[4])
+    ctx.sc_sweep(*args, exit_I=ex, J=torch.zeros_like(args[0]), noalloc=noalloc, **geo)
+    over = list(args)
+    over[4] = args[4].clone()
+    ctx.sc_sweep(*over, exit_I=over[4], J=torch.zeros_like(args[0]), noalloc=noalloc, **geo)
+    torch.cuda.synchronize()
+    assert float((over[4] - ex).abs().max()) <= 1e-6 * float(ex.abs().max())
