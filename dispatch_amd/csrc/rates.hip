@@ -113,7 +113,8 @@ struct RatesArgs {
   float wmu, wtot;
   float *gij, *gji;
   const float *tab;
-  int lchunk, nchunk, ncp;  // a lane's run of lines, the runs per cell, cells per run padded to 256
+  int lchunk, nchunk;       // a lane's run of lines, the runs per cell
+  uint32_t ncp;             // cells per run, padded to whole workgroups
 };
 
 // Lane (c, k): cell c, lines [k * lchunk, (k + 1) * lchunk), consecutive lanes on
@@ -133,9 +134,11 @@ __global__ void __launch_bounds__(kRateThreads) bb_rates_kernel(const RatesArgs 
   extern __shared__ float tab[];
   load_tables(tab, a.tab);
   const float *TGX = tab, *TH2X = tab + QLG_NX + 1;
-  const int base = blockIdx.x * blockDim.x;  // the lane count fits int32 (checked at launch)
-  const int k = base / a.ncp, c = base - k * a.ncp + threadIdx.x;
-  if (k >= a.nchunk || c >= a.ncell) return;
+  const uint32_t base = blockIdx.x * blockDim.x;  // the lane count fits 32 bits (checked at launch)
+  const int k = (int)(base / a.ncp);
+  const uint32_t cell = base - k * a.ncp + threadIdx.x;
+  if (k >= a.nchunk || cell >= (uint32_t)a.ncell) return;
+  const int c = (int)cell;
   const int nc = a.ncell;
   const bool split_pre = a.largest && a.precond;
   const float idf = a.inv_df[c], vpr = a.vproj[c], ekt = a.e_kT[c];
@@ -445,7 +448,8 @@ struct WinArgs {
   float floor_frac;
   int suppress;
   unsigned long long *n_floored;
-  int fchunk, nchunk, ncp;  // a lane's run of frequencies, the runs per cell, cells per run padded to 256
+  int fchunk, nchunk;       // a lane's run of frequencies, the runs per cell
+  uint32_t ncp;             // cells per run, padded to whole workgroups
 };
 
 // convert_to_work_units, the split tracking seeded with the continuum as contribution
@@ -612,9 +616,11 @@ __global__ void __launch_bounds__(kWinThreads) window_opacity_kernel(const WinAr
   // lane (c, k): cell c, frequencies [k * fchunk, (k + 1) * fchunk); consecutive lanes
   // take consecutive cells of one run, each run's cells padded to whole workgroups so
   // that k is the workgroup's
-  const int base = blockIdx.x * blockDim.x;  // the lane count fits int32 (checked at launch)
-  const int k = base / w.ncp, c = base - k * w.ncp + threadIdx.x;
-  if (k >= w.nchunk || c >= a.ncell) return;
+  const uint32_t base = blockIdx.x * blockDim.x;  // the lane count fits 32 bits (checked at launch)
+  const int k = (int)(base / w.ncp);
+  const uint32_t cell = base - k * w.ncp + threadIdx.x;
+  if (k >= w.nchunk || cell >= (uint32_t)a.ncell) return;
+  const int c = (int)cell;
   const int f_lo = k * w.fchunk, f_hi = min(a.nf, f_lo + w.fchunk);
   if (f_lo >= f_hi) return;
   const unsigned long long floored =
@@ -676,10 +682,14 @@ __global__ void __launch_bounds__(256) bf_rates_kernel(const BfArgs a) {
 // every cell's byte offset within one frequency fits 32 bits (4-byte elements)
 bool offsets32(int64_t ncell, int64_t sc) { return sc < (int64_t)1 << 30 && (ncell - 1) * sc < (int64_t)1 << 30; }
 
+// whether `nchunk` runs of the cells are within the lanes of one launch (the cells of
+// each padded to 256: a workgroup's own padding is beside that and below 2^32)
+bool lanes_fit(int64_t ncell, int64_t nchunk) { return (ncell + 255) / 256 * 256 * nchunk <= (int64_t)INT32_MAX; }
+
 template <typename K, typename A>
-int launch_cells(m3drt_ctx *ctx, K kern, const A &a, int ncell, size_t lds, int threads = 256) {
+int launch_cells(m3drt_ctx *ctx, K kern, const A &a, int64_t ncell, size_t lds, int threads = 256) {
   if (lds) M3DRT_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  hipLaunchKernelGGL(kern, dim3((ncell + threads - 1) / threads), dim3(threads), lds, ctx->stream, a);
+  hipLaunchKernelGGL(kern, dim3((unsigned)((ncell + threads - 1) / threads)), dim3(threads), lds, ctx->stream, a);
   M3DRT_HIP(hipGetLastError());
   return M3DRT_OK;
 }
@@ -718,11 +728,11 @@ int bb_rates(m3drt_ctx *ctx, const m3drt_bb_rates_args *r, const float *chi_cont
   nchunk = std::max(1, std::min(nchunk, r->nline));
   a.lchunk = (r->nline + nchunk - 1) / nchunk;
   a.nchunk = std::max(1, (r->nline + a.lchunk - 1) / std::max(1, a.lchunk));
-  a.ncp = (int)(((int64_t)r->ncell + kRateThreads - 1) / kRateThreads * kRateThreads);
+  a.ncp = (uint32_t)(((int64_t)r->ncell + kRateThreads - 1) / kRateThreads * kRateThreads);
   const int64_t lanes = (int64_t)a.ncp * a.nchunk;
-  if (lanes > (int64_t)INT32_MAX) return set_error(M3DRT_ELIMIT, "m3drt_bb_rates: too many points");
+  if (!lanes_fit(r->ncell, a.nchunk)) return set_error(M3DRT_ELIMIT, "m3drt_bb_rates: too many points");
   const size_t lds = 2 * (QLG_NX + 1) * sizeof(float);
-  auto run = [&](auto kern) { return launch_cells(ctx, kern, a, (int)lanes, lds, kRateThreads); };
+  auto run = [&](auto kern) { return launch_cells(ctx, kern, a, lanes, lds, kRateThreads); };
   if (offsets32(r->ncell, r->sc)) return chi_cont ? run(bb_rates_kernel<true, uint32_t>) : run(bb_rates_kernel<false, uint32_t>);
   return chi_cont ? run(bb_rates_kernel<true, int64_t>) : run(bb_rates_kernel<false, int64_t>);
 }
@@ -792,10 +802,10 @@ int window_opacity(m3drt_ctx *ctx, const m3drt_bb_opacity_args *r, const m3drt_w
   nchunk = std::max(1, std::min(nchunk, r->nf / 64));
   w.fchunk = (r->nf + nchunk - 1) / nchunk;
   w.nchunk = (r->nf + w.fchunk - 1) / w.fchunk;
-  w.ncp = (int)(((int64_t)r->ncell + kWinThreads - 1) / kWinThreads * kWinThreads);
+  w.ncp = (uint32_t)(((int64_t)r->ncell + kWinThreads - 1) / kWinThreads * kWinThreads);
   const int64_t lanes = (int64_t)w.ncp * w.nchunk;
-  if (lanes > (int64_t)INT32_MAX) return set_error(M3DRT_ELIMIT, "m3drt_window_opacity: too many points");
-  auto run = [&](auto kern) { return launch_cells(ctx, kern, w, (int)lanes, lds, kWinThreads); };
+  if (!lanes_fit(r->ncell, w.nchunk)) return set_error(M3DRT_ELIMIT, "m3drt_window_opacity: too many points");
+  auto run = [&](auto kern) { return launch_cells(ctx, kern, w, lanes, lds, kWinThreads); };
   const bool track = r->flags & M3DRT_BBOP_TRACK;
   if (offsets32(r->ncell, r->sc)) {
     if (track) return run(window_opacity_kernel<true, false, uint32_t>);
