@@ -128,7 +128,11 @@ struct RatesArgs {
 // windows mostly hold one line at a frequency, so this replaces 24 B a point, written
 // by the opacity pass and read here, by the 4 B of the continuum.  On the 432 000-cell
 // window of 2400 frequencies, with the threads above: opacity 12.8 -> 4.4 ms (20 B a
-// point, 4.7 TB/s), rates 9.9 -> 6.8 ms (32 B a point, 4.9 TB/s: HBM-bound).
+// point, 4.7 TB/s), rates 9.9 -> 6.8 ms (32 B a point, 4.9 TB/s: HBM-bound).  With n
+// lines at a frequency every one of them forms the n - 1 others: opacity and rates of
+// 216 000 cells x 1200 frequencies with 1 / 1.5 / 2 / 3 / 4 / 8 lines at a frequency
+// 2.9 / 5.4 / 8.1 / 15.1 / 24.7 / 95 ms, with the arrays 4.8 / 6.6 / 8.6 / 11.4 / 14.3 /
+// 26.2.  (The NLTE driver's windows hold one line at a frequency.)
 template <bool RETRACK, typename O>
 __global__ void __launch_bounds__(kRateThreads) bb_rates_kernel(const RatesArgs a) {
   extern __shared__ float tab[];

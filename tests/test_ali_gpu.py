@@ -169,6 +169,69 @@ def test_rates_with_the_tracking_formed_again(ctx, kw, overlap, off):
         assert torch.equal(a, b), (what, float((a - b).abs().max()))
 
 
+@pytest.mark.parametrize("layout", ["native", "reference"])
+@pytest.mark.parametrize("offs,scat,flags", [(True, False, False), (False, True, False), (False, False, True),
+                                             (True, True, True)])
+def test_tracking_formed_again_in_every_form(ctx, layout, offs, scat, flags):
+    """The same comparison for lines that blend, with lower levels off their term's
+    (lower_off, an exponential a line and cell), line scattering, psi flags read and
+    raised, and both layouts: chi, S, the rate sums and the raised flags bit for bit."""
+    from dispatch_amd import synth
+    from dispatch_amd.ali import NlteProblem
+    p = NlteProblem(ctx, small(nq=50, lines_per_window=6))
+    g = torch.Generator(device="cuda").manual_seed(7)
+    p.b.mul_(torch.exp(0.3 * torch.randn(p.b.shape, generator=g, dtype=torch.float64, device="cuda")))
+    w = p.windows[0]
+    l0, l1, nf, nc = w.lines[0], w.lines[-1] + 1, w.nf, p.ncell
+    nl = l1 - l0
+    print(f"tracking formed again {layout} lower_off={offs} scat={scat} flags={flags}", flush=True)
+    const = _overlapping(p, w, 9)
+    cover = torch.zeros(nf, dtype=torch.int32)
+    for a, b in zip(const["iblue"].tolist(), const["ired"].tolist()):
+        cover[a - 1:b] += 1
+    assert int(cover.max()) > 1
+    if offs:
+        const["lower_off"] = (0.1 * torch.randn(nl, generator=g, device="cuda")).contiguous()
+        const["lower_off"][::3] = 0.0
+    lay = (lambda t: t) if layout == "native" else (lambda t: t.T.contiguous())
+    d = dict(const, vproj=(p.vz * (p.vec[0][2] / synth.C_LIGHT)).float().contiguous(), b=p.b, nstar=p.nstar,
+             pop_ratio=p.pop_ratio, inv_df=p.inv_df, e_kT=p.e_kT32, adamp=p.adamp[l0:l1])
+    rnd = lambda: torch.rand((nf, nc), generator=g, device="cuda")
+    cont, B, beta = lay(w.chi_c), lay(w.Bnu), lay(w.beta)
+    I, Irem, esc = lay(rnd() * w.Bnu), lay(rnd() * w.Bnu), lay(rnd())
+    extra = {}
+    if scat:
+        extra.update(chi_scat=lay(0.1 * rnd() * w.chi_c), dJnu=lay(rnd() * w.Bnu))
+    raised = torch.randint(0, 1 << 20, (2, nc), generator=g, device="cuda", dtype=torch.int32)
+    if flags:
+        extra.update(ntrans=torch.arange(30, 30 + nl, dtype=torch.int32, device="cuda"),
+                     psi_flags_in=torch.randint(0, 1 << 30, (2, nc), generator=g, device="cuda", dtype=torch.int32))
+    out = []
+    for retrack in (False, True):
+        chi, S = torch.empty_like(cont), torch.empty_like(cont)
+        sp = {}
+        if not retrack:
+            sp = {k: torch.empty_like(cont) for k in ("split_opac1", "split_opac2", "split_chi1", "split_chi2")}
+            sp.update({k: torch.empty(cont.shape, dtype=torch.int32, device="cuda") for k in ("split_id", "split_chi_id")})
+        ctx.window_opacity(d, cont, B, beta, chi, S, split=None if retrack else sp, split_offset=5, track=retrack,
+                           layout=layout)
+        Psi = torch.where(I < 0.05 * B, torch.zeros_like(chi), esc / chi.abs())
+        gij, gji = torch.zeros((nl, nc), device="cuda"), torch.zeros((nl, nc), device="cuda")
+        up = raised.clone()
+        parts = dict(sp, Irem=Irem, escape=esc, chi=chi, **extra, **({"psi_flags_out": up} if flags else {}))
+        dr = dict(d, Inu=I, Psi=Psi, Bnu=B, beta=beta)
+        if retrack:
+            ctx.bb_rates_window(dr, cont, 0.3, 1.0, gij, gji, own_norm=True, split=parts, split_offset=5, layout=layout)
+        else:
+            ctx.bb_rates(dr, 0.3, 1.0, gij, gji, precond=True, largest=True, own_norm=True, split=parts, split_offset=5,
+                         layout=layout)
+        out.append((chi, S, gij, gji, up))
+    torch.cuda.synchronize()
+    assert float(out[0][2].abs().max()) > 0 and (not flags or not torch.equal(out[0][4], raised))
+    for a, b, what in zip(*out, ("chi", "S", "gamma_ij", "gamma_ji", "raised flags")):
+        assert torch.equal(a, b), (what, float((a.double() - b.double()).abs().max()))
+
+
 def test_tracking_flags_that_contradict_are_refused(ctx):
     """Tracking arrays together with M3DRT_BBOP_TRACK would stay unwritten, and
     m3drt_bb_opacity has no such form: both are errors, and nothing is written."""
