@@ -232,9 +232,10 @@ def adjoint_leg(ctx, args):
     2048 frequencies, 12 lines of 4 elements).  Forwards, one launch per ray and
     nothing kept: the 12 upward rays' exit planes the flux loss needs, and the
     24-ray formal solution with J.  Gradient of the flux chi^2: the checkpointed
-    forward of the 12 upward rays (patches of 23 planes, exit planes kept), the
-    backward (each patch recomputed from its checkpoint and swept in reverse), and
-    the chain to the 4 log abundances.  Checked against FP64 central differences
+    forward of the 12 upward rays (patches of 23 planes, exit planes kept, and the
+    intensity cubes of as many rays as RaySet.keep's "auto" allows), the backward (each
+    patch swept in reverse, of the other rays after its recomputation from the
+    checkpoint), and the chain to the 4 log abundances.  Checked against FP64 central differences
     (h = 1e-3 dex) unless --no-adjoint-fd."""
     import torch
     from dispatch_amd.fit import FitProblem

@@ -646,7 +646,7 @@ int run_fast(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const m3drt_sweep_bufs *
   const int want = lenv ? atoi(lenv) : 0;
   auto max_threads = [](int l) { return l >= 30 ? 512 : l >= 20 ? 768 : 1024; };
   int L = 0;
-  if (!want && !L && cpl == 1 && ny % 20 == 0 && ny / 20 >= 2 && (ny / 20) * nx >= 512 && (ny / 20) * nx <= 768) L = 20;
+  if (!want && cpl == 1 && ny % 20 == 0 && ny / 20 >= 2 && (ny / 20) * nx >= 512 && (ny / 20) * nx <= 768) L = 20;
   // Where the pairs and S of three workgroups fit one CU's LDS, a strip of 15 (or 20)
   // rows that still gives a workgroup more than three waves: four rows of loads in
   // flight instead of three, three workgroups per CU.  On the 60 x 60 plane the
@@ -685,8 +685,12 @@ int run_fast(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const m3drt_sweep_bufs *
     int best = 0;
     for (int c : kRag) {
       const int t = (ny + c - 1) / c * nx, cap = c <= 2 ? 2048 : c <= 4 ? 1536 : c <= 12 ? 1024 : 768;
-      // (with PsiJ strips of 20 spill: 556 us against the general kernel's 500 on
-      // 118 x 110 x 250, 1085 against 1002 on 117 x 113 x 500, 23 planes)
+      // (With PsiJ strips of 20 are left out.  Where S comes from the cache they spill and
+      // lose: 374 us against the general kernel's 343 on 117 x 113 x 250, 15 planes; with S
+      // in LDS they would win 4 % where nothing shorter fits: 437 against 456 on
+      // 117 x 101 x 250, 23 planes.  Other forms that spill a few registers with S from the
+      // cache win: strips of 12 with PsiJ 297 against 322 on 32 x 383 x 250, of 20 with J
+      // alone 246 against 301 on 117 x 113 x 250.)
       if (c == 20 && get_rates && b->PsiJ && !rwant) continue;
       if (c + 2 > ny || t > max_threads(c) || lds > (size_t)ctx->lds_max || (rwant && c != rwant)) continue;
       const int wgs = std::max(1, std::min(cap / t, (int)((size_t)ctx->lds_max / lds)));
