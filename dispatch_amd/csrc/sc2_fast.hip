@@ -710,8 +710,21 @@ int run_fast(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const m3drt_sweep_bufs *
   // (From 8 frequencies on; fewer were not measured and keep the strip that divides.)
   // Strips of 4 that tile ny but fit a CU at most twice and leave another round of
   // workgroups: the longer ones (48 x 48 x 1000 265 with 12 against 312).
-  const int64_t pts = (int64_t)nx * ny * d->nf;
-  const bool rag = Lr && (!L || rwant || (Lr < L && d->nf >= 8 && pts < (L == 4 ? 180000 : 1300000)) ||
+  // Cubes with the frequencies at unit stride read a cache line a value, and a strip of 2
+  // reads 5 rows of them for 2: strips of 4 that tile ny stay on planes of 760 cells and
+  // more (20 planes, us, 4 against 2: 28 x 28 x 48 74 / 78, 20 x 40 x 48 75 / 80; 24 x 24 x
+  // 48 65 / 58) and from 76 000 points (20 x 20 x 300 106 / 111, with PsiJ 12 x 12 x 700
+  // 101 / 110); and where none tiles it the general kernel, if it takes a row a thread (a
+  // single strip of 15 is slower: 30 x 15 x 100 142 / 52), stays between
+  // 100 and 768 cells but for J or I alone on fewer than 12 000 points (general against 2:
+  // 15 x 17 x 120 35 / 41, 23 x 25 x 48 57 / 61, 15 x 22 x 16 36 / 32, with PsiJ 11 x 14 x
+  // 120 34 / 40; 9 x 7 x 120 30 / 26, 41 x 19 x 48 91 / 78, 29 x 31 x 120 103 / 93).
+  const int64_t pts = (int64_t)nx * ny * d->nf, cells = (int64_t)nx * ny;
+  const bool apart_x = d->cs_x != 1;
+  const bool odd = !apart_x || cells > 768 || cells <= 100 || sc2_general_fixed_outputs(d, b) ||
+                   (!spl && !(get_rates && b->PsiJ) && pts < 12000);
+  const int64_t few = L != 4 ? 1300000 : !apart_x ? 180000 : cells < 760 ? 76000 : 0;
+  const bool rag = Lr && (rwant || (!L && odd) || (L && Lr < L && d->nf >= 8 && pts < few) ||
                           (L == 4 && Lr > 4 && ny / 4 * nx > 512));
   // the kernel that would take the call without them: the general one (strips of 24 and
   // 30 have no split outputs), or strips that divide ny

@@ -532,3 +532,33 @@ def test_exit_plane_alone_has_the_cubes_bits(ctx, nf, nx, ny, nz):
     assert float(alone.abs().max()) > 0
     assert torch.equal(beside, I[-1])
     assert torch.equal(alone, beside), float((alone - beside).abs().max())
+
+
+# the frequencies at unit stride on planes below the plane-by-plane kernel's: strips of 2
+# only where they are the faster ones (measured lines beside the rule), seen in what the
+# library reports of the form it takes
+@pytest.mark.parametrize("nx,ny,nf,psi,want", [
+    (24, 24, 48, False, "strip 2"), (28, 28, 48, False, "strip 4"), (62, 16, 58, False, "strip 4"),
+    (20, 20, 300, False, "strip 4"), (12, 30, 60, False, "strip 2"), (15, 22, 225, False, "general"),
+    (15, 17, 120, False, "general"), (15, 22, 16, False, "strip 2"), (11, 14, 120, True, "general"),
+    (9, 7, 120, False, "strip 2"), (41, 19, 48, False, "strip 2"), (29, 31, 40, True, "strip 2"), (30, 15, 100, False, "strip 2"),
+])
+def test_strips_of_strided_rows(ctx, capfd, monkeypatch, nx, ny, nf, psi, want):
+    monkeypatch.setenv("M3DRT_VERBOSE", "1")
+    g = torch.Generator(device="cuda").manual_seed(nx)
+    r = lambda *s: torch.rand(s, generator=g, device="cuda") + 0.5
+    nz = 3
+    chi, S, gh = r(nz, ny, nx, nf) * 1e-7, r(nz, ny, nx, nf), [r(ny, nx, nf) * 1e-7, r(ny, nx, nf), r(ny, nx, nf)]
+    c5, cu, g5 = r(nz, ny, nx) * 1e-7, r(nz, ny, nx) * 1e-7, r(ny, nx) * 1e-7
+    geo = dict(dir=1, ds=(50e5, 50e5, 10e5), vec=(0.3, -0.4, 0.866), wj=0.25)
+    zero = lambda t: dict(J=torch.zeros_like(t), **(dict(PsiJ=torch.zeros_like(t), get_rates=True) if psi else {}))
+    out = zero(chi)
+    ctx.sc_sweep(chi, S, *gh, c5, cu, g5, layout="reference", **geo, **out)
+    torch.cuda.synchronize()
+    said = capfd.readouterr().err
+    assert ("sc2 fast" not in said) if want == "general" else (want + "," in said), said
+    nat, pla = (lambda t: t.permute(0, 3, 1, 2).contiguous()), (lambda t: t.permute(2, 0, 1).contiguous())
+    ref = zero(nat(chi))
+    ctx.sc_sweep(nat(chi), nat(S), *[pla(t) for t in gh], c5, cu, g5, **geo, **ref)
+    for k in ("J", "PsiJ")[:1 + psi]:
+        assert float((nat(out[k]) - ref[k]).abs().max()) <= 1e-6 * float(ref[k].abs().max()), k
