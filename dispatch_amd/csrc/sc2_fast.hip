@@ -724,7 +724,21 @@ int run_fast(m3drt_ctx *ctx, const m3drt_sweep_desc *d, const m3drt_sweep_bufs *
   const bool odd = !apart_x || cells > 768 || cells <= 100 || sc2_general_fixed_outputs(d, b) ||
                    (!spl && !(get_rates && b->PsiJ) && pts < 12000);
   const int64_t few = L != 4 ? 1300000 : !apart_x ? 180000 : cells < 760 ? 76000 : 0;
-  const bool rag = Lr && (rwant || (!L && odd) || (L && Lr < L && d->nf >= 8 && pts < few) ||
+  // Longer strips that divide ny on few points.  Where the last-level cache holds the cubes,
+  // a workgroup's plane takes about its rows a thread times its waves a SIMD, and strips of
+  // 12 are replaced only where that falls, or stays for outputs other than I alone (15
+  // planes, 40 to 79 frequencies, us, 12 against 8: 100 x 60 72 / 80 J, 69 / 79 I; 96 x 60
+  // 74 / 74, 69 / 71; 84 x 84 93 / 86, 90 / 84).  Where it does not (us a plane): strips of
+  // 12 where that stays (96 x 60 x 79 4.43 / 4.65 J), and without PsiJ strips of 15 and 20
+  // on planes above 3700 cells whose columns do not fill the waves (51 x 105 x 79 5.04 with
+  // 15 against 5.51 with 8, 75 x 75 x 79 5.02 / 5.32; 64 x 75 x 79 4.65 / 4.07, 60 x 60 x 79
+  // 3.76 with 15 against 3.41 with 4, with PsiJ 51 x 105 x 79 8.02 / 7.28).
+  const bool cached = 12 * pts * nz <= (int64_t)192 << 20;
+  auto turns = [&](int c) { return c * ((((ny + c - 1) / c * nx + 63) / 64 + 3) / 4); };
+  bool shorter = Lr && Lr < L;
+  if (shorter && L == 12) shorter = turns(Lr) < turns(12) + (cached && (b->J || spl) ? 1 : 0);
+  if (shorter && L > 12 && !cached && !(get_rates && b->PsiJ)) shorter = cells < 3700 || nx % 64 == 0;
+  const bool rag = Lr && (rwant || (!L && odd) || (shorter && d->nf >= 8 && pts < few) ||
                           (L == 4 && Lr > 4 && ny / 4 * nx > 512));
   // the kernel that would take the call without them: the general one (strips of 24 and
   // 30 have no split outputs), or strips that divide ny

@@ -562,3 +562,19 @@ def test_strips_of_strided_rows(ctx, capfd, monkeypatch, nx, ny, nf, psi, want):
     ctx.sc_sweep(nat(chi), nat(S), *[pla(t) for t in gh], c5, cu, g5, **geo, **ref)
     for k in ("J", "PsiJ")[:1 + psi]:
         assert float((nat(out[k]) - ref[k]).abs().max()) <= 1e-6 * float(ref[k].abs().max()), k
+
+
+@pytest.mark.parametrize("nx,ny,nz,out,want", [
+    (100, 60, 2, "J", "strip 12"), (100, 60, 2, "I_out", "strip 12"), (96, 60, 2, "J", "strip 8"), (96, 60, 80, "J", "strip 12"),
+    (96, 60, 2, "I_out", "strip 12"), (84, 84, 2, "I_out", "strip 8"), (51, 105, 2, "J", "strip 8"),
+    (51, 105, 100, "J", "strip 15"), (64, 75, 110, "J", "strip 8"), (60, 60, 150, "J", "strip 4")])
+def test_longer_strips_stay_where_shorter_ones_lose(ctx, capfd, monkeypatch, nx, ny, nz, out, want):
+    monkeypatch.setenv("M3DRT_VERBOSE", "1")
+    nf = 40
+    r = lambda *s: torch.rand(s, device="cuda") + 0.5
+    chi = r(nz, nf, ny, nx) * 1e-7
+    ctx.sc_sweep(chi, r(nz, nf, ny, nx), r(nf, ny, nx) * 1e-7, r(nf, ny, nx), r(nf, ny, nx), r(nz, ny, nx) * 1e-7,
+                 r(nz, ny, nx) * 1e-7, r(ny, nx) * 1e-7, dir=1, ds=(50e5, 50e5, 10e5), vec=(0.3, -0.4, 0.866), wj=0.25,
+                 **{out: torch.zeros_like(chi)})
+    torch.cuda.synchronize()
+    assert want + "," in capfd.readouterr().err
